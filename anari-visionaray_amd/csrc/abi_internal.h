@@ -12,8 +12,8 @@ struct vrt_context_s {
   hipStream_t stream = nullptr;
   hipEvent_t t0 = nullptr, t1 = nullptr;
   int num_cus = 0;
-  // work-queue counters of the persistent path tracer: two sets of 8, used
-  // alternately; each launch clears the set the next launch uses
+  // work-queue counters of the persistent kernels: two sets of 8 (kWorkQueueWords
+  // words each), used alternately; each launch clears the set the next launch uses
   uint32_t *queues = nullptr;
   int queue_parity = 0;
   // device address of the library's file-scope queue counters on this

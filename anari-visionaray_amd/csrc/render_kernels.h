@@ -5,6 +5,11 @@
 
 namespace vrt {
 
+// work-queue counters of the persistent kernels: one per XCD, 256 B apart so
+// that no two share a cache line
+constexpr int kWorkQueues = 8;
+constexpr int kWorkQueueWords = kWorkQueues * 64;
+
 hipError_t launch_raycast(const KScene &sc, const KCamera &cam, const KParams &P, const KFrame &F,
                           uint32_t *queues, uint32_t *queues_next, int num_cus, hipStream_t s);
 // persistent path tracer: `blocks` workgroups (a multiple of 8) drain the

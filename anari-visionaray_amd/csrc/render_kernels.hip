@@ -51,10 +51,54 @@ __device__ inline float rnd(uint32_t &s) {
 
 // ---------------------------------------------------------------------------
 // Work queues: the persistent kernels cut the image into 8 parts, one per
-// XCD (the hardware places workgroup b on XCD b % 8), each drained from an
-// atomic counter
+// XCD (the hardware places workgroup b on XCD b % 8).  Every wave's first
+// units are its own by position (no atomic); the units after those of the
+// `first` resident waves of a queue are claimed from the queue's counter.
+//
+// Atomics from 8 XCDs on one cache line are executed one after another,
+// about 10 ns each, so each counter has a line of its own, and a wave whose
+// queue is drained reads all 8 counters with one load and goes to a queue
+// that has units left, instead of asking each with an atomic (8 x 3072 waves
+// x 10 ns = 0.25 ms per frame, whatever its size).
 // ---------------------------------------------------------------------------
-constexpr int kQueues = 8;
+constexpr int kQueues = kWorkQueues;
+constexpr int kQueueStride = kWorkQueueWords / kWorkQueues;
+
+__device__ inline void clear_queues(uint32_t *queues) {
+  if (blockIdx.x == 0 && threadIdx.x < kQueues) queues[threadIdx.x * kQueueStride] = 0u;
+}
+
+// `step` units for the wave from queue q or, once that is drained, from the
+// next queue with units left (q then names it): the index of the first one
+// in queue q, or kDrained when nothing is left anywhere.  Units below `first`
+// are not the counters' to give; band(i) is the number of units of queue i.
+// The counters only grow, so the loop ends: a failed claim on a queue that
+// had units left when it was read means that other waves took them.
+constexpr uint32_t kDrained = 0xFFFFFFFFu;
+
+template <class Band>
+__device__ inline uint32_t queue_claim(uint32_t *queues, int &q, uint32_t step, uint32_t first,
+                                       const Band &band) {
+  const int lane = int(threadIdx.x) & 63;
+  bool ask = first < band(q);  // else the queue held no more than the first units
+  while (true) {
+    if (ask) {
+      uint32_t k = 0;
+      if (lane == 0) k = atomicAdd(&queues[q * kQueueStride], step);
+      k = first + uint32_t(__builtin_amdgcn_readfirstlane(int(k)));
+      if (k < band(q)) return k;
+    }
+    const int i = (q + 1 + lane) & (kQueues - 1);
+    bool some = false;
+    if (lane < kQueues && first < band(i))
+      some = first + __hip_atomic_load(&queues[i * kQueueStride], __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT) < band(i);
+    const unsigned long long m = __ballot(some);
+    if (m == 0ull) return kDrained;
+    q = (q + __ffsll(m)) & (kQueues - 1);
+    ask = true;
+  }
+}
 
 // ---------------------------------------------------------------------------
 // Rays / boxes
@@ -1714,24 +1758,20 @@ __global__ void __launch_bounds__(256)
   stage_tf(sc, s_tf);  // (its barrier also publishes s_pow and the nodes)
   // clear the counters the next launch will use (the current ones were
   // cleared by the previous launch)
-  if (blockIdx.x == 0 && threadIdx.x < kQueues) queues_next[threadIdx.x] = 0u;
+  clear_queues(queues_next);
   const int lane = int(threadIdx.x) & 63;
   const int ntx = (F.width + 7) >> 3;
   const uint32_t ntiles = uint32_t(ntx) * uint32_t((F.height + 7) >> 3);
   uint32_t lookups = 0;
   int q = int(blockIdx.x) & (kQueues - 1);
-  for (int tries = 0; tries < kQueues;) {
-    const uint32_t lo = ntiles * uint32_t(q) / kQueues;
-    const uint32_t hi = ntiles * uint32_t(q + 1) / kQueues;
-    uint32_t k = 0;
-    if (lane == 0) k = atomicAdd(&queues[q], 1u);
-    k = __shfl(k, 0, 64);
-    if (lo + k >= hi) {  // band drained: help the next one
-      q = (q + 1) & (kQueues - 1);
-      ++tries;
-      continue;
-    }
-    const int tile = int(lo + k);
+  auto first_of = [&](int i) { return uint32_t(uint64_t(ntiles) * uint32_t(i) / kQueues); };
+  auto band = [&](int i) { return first_of(i + 1) - first_of(i); };
+  // the grid is a multiple of 8 workgroups: `waves` of them start on each queue
+  const uint32_t waves = gridDim.x / kQueues * 4u;
+  uint32_t k = (blockIdx.x / kQueues) * 4u + uint32_t(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+  if (k >= band(q)) k = queue_claim(queues, q, 1u, waves, band);
+  for (; k != kDrained; k = queue_claim(queues, q, 1u, waves, band)) {
+    const int tile = int(first_of(q) + k);
     const int x = (tile % ntx) * 8 + (lane & 7), y = (tile / ntx) * 8 + (lane >> 3);
     raycast_pixel<ANYF, SHADE, SURF, INST>(sc, cam, P, F, x, y, s_tf, s_pow, lookups);
   }
@@ -2347,7 +2387,7 @@ __global__ void __launch_bounds__(256, 3)
   stage_tf(sc, s_tf);  // (its barrier also publishes the nodes)
   // clear the counters the next launch will use (the current ones were
   // cleared by the previous launch)
-  if (blockIdx.x == 0 && threadIdx.x < kQueues) queues_next[threadIdx.x] = 0u;
+  clear_queues(queues_next);
   // fraction of paths that become training paths: the per-frame training
   // budget over the previous frame's count of paths reaching vertex 2
   float p_train = 0.f;
@@ -2376,8 +2416,18 @@ __global__ void __launch_bounds__(256, 3)
   st.pixel = -1;
   uint32_t lookups = 0, hit_samples = 0;
   int q = int(blockIdx.x) & (kQueues - 1);  // wave-uniform queue
-  int qtries = 0;
-  uint32_t pool_base = 0, pool_left = 0;    // wave-uniform local pool
+  // pixels of queue i: the chunks c = i, i+8, ... times 1024 pixels
+  auto band = [&](int i) {
+    return ((nch + kQueues - 1 - uint32_t(i)) / kQueues) << (2 * kChunkLog2);
+  };
+  // the grid is a multiple of 8 workgroups: `waves` of them start on each
+  // queue, each with the 64 pixels of its position
+  const uint32_t waves = gridDim.x / kQueues * 4u;
+  // wave-uniform local pool
+  uint32_t pool_base = 64u * ((blockIdx.x / kQueues) * 4u +
+                              uint32_t(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)));
+  uint32_t pool_left = pool_base < band(q) ? 64u : 0u;
+  bool drained = false;
   int px = 0, py = 0;
 
   // chain: this lane's bounce continues with its shadow / AO rays; while any
@@ -2390,20 +2440,12 @@ __global__ void __launch_bounds__(256, 3)
     unsigned long long idle = chained ? 0ull : __ballot(st.pixel < 0);
     if (P.refill_min > 1 && __popcll(idle) < P.refill_min && __ballot(st.pixel >= 0) != 0ull)
       idle = 0ull;  // refill later, for more lanes at once
-    while (idle && qtries < kQueues) {
+    while (idle && !drained) {
       if (pool_left == 0) {
-        // pixels of queue q: the chunks c = q, q+8, ... times 1024 pixels
-        const uint32_t band = ((nch + kQueues - 1 - uint32_t(q)) / kQueues) << (2 * kChunkLog2);
-        uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(&queues[q], 64u);
-        base = __shfl(base, 0, 64);
-        if (base >= band) {
-          q = (q + 1) & (kQueues - 1);
-          ++qtries;
-          continue;
-        }
-        pool_base = base;
-        pool_left = min(64u, band - base);
+        pool_base = queue_claim(queues, q, 64u, 64u * waves, band);
+        drained = pool_base == kDrained;
+        if (drained) break;
+        pool_left = 64u;  // (a band is a multiple of 64)
       }
       const uint32_t nidle = uint32_t(__popcll(idle));
       const uint32_t take = min(nidle, pool_left);
@@ -2428,7 +2470,7 @@ __global__ void __launch_bounds__(256, 3)
     if (!chained && __ballot(st.pixel >= 0) == 0ull) {
       // no lane holds a pixel: either every queue is drained, or the last
       // pool only covered padding pixels outside the image -- claim again
-      if (qtries >= kQueues) break;
+      if (drained) break;
       continue;
     }
 
@@ -3166,18 +3208,18 @@ hipError_t launch_pathtrace(const KScene &sc, const KCamera &cam, const KParams 
 
 // ---------------------------------------------------------------------------
 // Work-queue counters of vrt_pathtrace_noalloc: a file-scope device array
-// (two sets of kQueues words, 64 B) in place of the context's allocation.
+// (two sets of kWorkQueueWords) in place of the context's allocation.
 // Every GPU holds its own copy until the process ends; host code reaches it
 // only through the address hipGetSymbolAddress returns on that device.
 // Each call clears the set it claims from with a kernel (no memset node), so
 // the call may be captured into a graph; calls that overlap on one GPU share
 // the array and race.
 // ---------------------------------------------------------------------------
-constexpr int kScratchWords = 2 * kQueues;
+constexpr int kScratchWords = 2 * kWorkQueueWords;
 static __device__ __align__(256) uint32_t scratch[kScratchWords];
 
 __global__ void k_clear_words(uint32_t *p, int n) {
-  if (int(threadIdx.x) < n) p[threadIdx.x] = 0u;
+  for (int i = int(threadIdx.x); i < n; i += int(blockDim.x)) p[i] = 0u;
 }
 
 hipError_t static_queue_address(uint32_t **ptr) {
@@ -3190,10 +3232,10 @@ hipError_t static_queue_address(uint32_t **ptr) {
 hipError_t launch_pathtrace_static(const KScene &sc, const KCamera &cam, const KParams &P,
                                    const KFrame &F, int accumID, uint32_t *scratch_ptr,
                                    int blocks, hipStream_t s) {
-  hipLaunchKernelGGL(k_clear_words, dim3(1), dim3(64), 0, s, scratch_ptr, kScratchWords);
+  hipLaunchKernelGGL(k_clear_words, dim3(1), dim3(256), 0, s, scratch_ptr, kScratchWords);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  return launch_pathtrace(sc, cam, P, F, accumID, scratch_ptr, scratch_ptr + kQueues, blocks, s);
+  return launch_pathtrace(sc, cam, P, F, accumID, scratch_ptr, scratch_ptr + kWorkQueueWords, blocks, s);
 }
 
 hipError_t launch_taa_resolve(const KFrame &F, float alpha, hipStream_t s) {

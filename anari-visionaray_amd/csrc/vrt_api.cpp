@@ -389,8 +389,8 @@ int vrt_context_create(int device, vrt_context *out) {
   if (e == hipSuccess) e = hipEventCreate(&c->t0);
   if (e == hipSuccess) e = hipEventCreate(&c->t1);
   if (e == hipSuccess) e = hipDeviceGetAttribute(&c->num_cus, hipDeviceAttributeMultiprocessorCount, device);
-  if (e == hipSuccess) e = hipMalloc(&c->queues, 2 * 8 * sizeof(uint32_t));
-  if (e == hipSuccess) e = hipMemset(c->queues, 0, 2 * 8 * sizeof(uint32_t));
+  if (e == hipSuccess) e = hipMalloc(&c->queues, 2 * kWorkQueueWords * sizeof(uint32_t));
+  if (e == hipSuccess) e = hipMemset(c->queues, 0, 2 * kWorkQueueWords * sizeof(uint32_t));
   if (e == hipSuccess) e = vrt::static_queue_address(&c->static_queues);
   if (e != hipSuccess) {
     delete c;
@@ -687,8 +687,8 @@ int vrt_raycast(vrt_context ctx, const vrt_scene *scene, const vrt_camera *camer
   // the fixed-step marcher reads no majorants
   sc.maj_lds_bytes = 0;
   for (int i = 0; i < sc.num_volumes; ++i) sc.vol[i].maj_lds_offset = -1;
-  uint32_t *cur = ctx->queues + 8 * ctx->queue_parity;
-  uint32_t *nxt = ctx->queues + 8 * (1 - ctx->queue_parity);
+  uint32_t *cur = ctx->queues + kWorkQueueWords * ctx->queue_parity;
+  uint32_t *nxt = ctx->queues + kWorkQueueWords * (1 - ctx->queue_parity);
   VRT_HIP(launch_raycast(sc, cam, P, F, cur, nxt, ctx->num_cus, ctx->stream));
   ctx->queue_parity ^= 1;
   return VRT_OK;
@@ -764,8 +764,8 @@ int pathtrace_frame(vrt_context ctx, const vrt_scene *scene, const vrt_camera *c
     VRT_HIP(launch_pathtrace_static(sc, cam, P, F, accum_id, ctx->static_queues, blocks,
                                     ctx->stream));
   } else {
-    uint32_t *cur = ctx->queues + 8 * ctx->queue_parity;
-    uint32_t *nxt = ctx->queues + 8 * (1 - ctx->queue_parity);
+    uint32_t *cur = ctx->queues + kWorkQueueWords * ctx->queue_parity;
+    uint32_t *nxt = ctx->queues + kWorkQueueWords * (1 - ctx->queue_parity);
     VRT_HIP(launch_pathtrace(sc, cam, P, F, accum_id, cur, nxt, blocks, ctx->stream));
     ctx->queue_parity ^= 1;
   }
@@ -869,8 +869,8 @@ int vrt_pathtrace_nrc(vrt_context ctx, const vrt_scene *scene, const vrt_camera 
   plan_staged_nodes(sc, lds, per_cu);
   int blocks = std::max(1, ctx->num_cus) * per_cu;
   blocks = std::max(8, (blocks + 7) / 8 * 8);
-  uint32_t *cur = ctx->queues + 8 * ctx->queue_parity;
-  uint32_t *nxt = ctx->queues + 8 * (1 - ctx->queue_parity);
+  uint32_t *cur = ctx->queues + kWorkQueueWords * ctx->queue_parity;
+  uint32_t *nxt = ctx->queues + kWorkQueueWords * (1 - ctx->queue_parity);
   VRT_HIP(launch_pathtrace(sc, cam, P, F, accum_id, cur, nxt, blocks, ctx->stream, &N));
   ctx->queue_parity ^= 1;
   // answer the queries (count taken on the GPU), add the cache term, write

@@ -568,8 +568,8 @@ VRT_API int vrt_pathtrace(vrt_context ctx, const vrt_scene *scene,
 /* 'pathtrace' renderer, one frame, allocating nothing: no counterpart in the
  * reference.  For callers that cannot allocate device memory (code under HIP
  * graph capture, serving loops).  Same arguments, semantics and image as
- * vrt_pathtrace; the persistent kernel's work-queue counters (16 uint32) live
- * in a file-scope device array of the library instead of the context's
+ * vrt_pathtrace; the persistent kernel's work-queue counters (two sets of 8, 4 KB)
+ * live in a file-scope device array of the library instead of the context's
  * allocation, cleared by a kernel at the start of every call (no memset).
  * Each GPU holds one such array until the process ends, so calls that
  * overlap on one GPU (several contexts or streams) race; serialise them.
