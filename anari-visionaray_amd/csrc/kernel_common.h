@@ -41,7 +41,6 @@ struct KVolume {
   float cell_size;
   const float *bricks; // structured: brick records of 9^3 voxels (VRT_BRICK_FLOATS each)
   uint32_t nbx, nby;   // structured: bricks per x row, per y column
-  const float *leaves; // nanovdb: 512 values per leaf
   const float4 *tf;    // global copy of the table
   int tf_size;
   int tf_lds_offset;   // offset of this table in the block's LDS copy
@@ -58,16 +57,25 @@ struct KVolume {
   f3 tinv;             // transInv
   uint32_t obj_id, inst_id;
   f3 glo, ghi;         // majorant grid bounds in voxel space
-  // nanovdb: top table over 128^3 regions (>= 0 block index, < 0: -1 -
-  // index into nv_consts), blocks of 16^3 slot entries (>= 0 leaf index
-  // into `leaves`, else a constant), top origin (in 128-voxel units) / dims,
-  // world -> index map, filter
-  const int32_t *nv_top;
-  const int32_t *nv_blocks;
+  // nanovdb lookups: a table over the 8^3-voxel slots [nv_slo, nv_slo +
+  // nv_sn) whose entry is a record of 9^3 voxels in nv_recs (>= 0,
+  // VRT_BRICK_FLOATS each) or -1 - index into nv_consts (0: the background,
+  // also outside); with nv_rtop the table holds blocks of 16^3 slots, nv_slo
+  // and nv_sn count 128^3 regions and nv_rtop gives a region's block or
+  // constant.  World -> index map, filter
+  const float *nv_recs;
+  const int32_t *nv_tab;
+  const int32_t *nv_rtop;
   const float *nv_consts;
+  float nv_bg;
+  int nv_slo[3], nv_sn[3];
+  float nv_inv[9], nv_vec[3];
+  // nanovdb value ranges: top table over 128^3 regions (>= 0 block index,
+  // else a constant), value range of each slot of the blocks, top origin (in
+  // 128-voxel units) / dims
+  const int32_t *nv_top;
   const float *nv_slot_ranges;
   int nv_lo[3], nv_n[3];
-  float nv_inv[9], nv_vec[3];
   int filter;
   // unstructured: point-location grid (list start per grid cell, dims
   // product + 1 entries; tetrahedron copies of four float4 {x, y, z, value}

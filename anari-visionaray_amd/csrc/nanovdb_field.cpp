@@ -2,7 +2,7 @@
 // the GPU layout, replacing NanoVDBField::finalize's device copy of the
 // buffer (NanoVDBField.cpp:30-65).
 //
-// Layout on the device, two levels instead of NanoVDB's four:
+// The tree is first painted into two levels instead of NanoVDB's four:
 //  * a dense x-fastest top table over 128^3-voxel regions (the extent of a
 //    lower internal node) covering the grid's bounds plus one region of
 //    apron: a block index (>= 0) where a lower node exists, else -1 - c for
@@ -11,9 +11,16 @@
 //    (>= 0) or -1 - c for a lower-node tile;
 //  * the leaf values, 512 floats per leaf in NanoVDB's in-leaf order
 //    (i&7)<<6 | (j&7)<<3 | (k&7).
-// A lookup is two table reads and one value read instead of a root tile
-// search plus three node levels; grids with huge tiles stay small because a
-// tile costs one top entry.
+// Grids with huge tiles stay small because a tile costs one top entry.
+//
+// From these the GPU builds what lookups read: a table with one entry per
+// 8^3 slot of the box that holds anything but background, and, for each slot
+// whose 9^3 voxels (its own and the first layers of its 7 upper neighbours)
+// are not one constant, a record of these voxels (VRT_BRICK_FLOATS floats, x
+// fastest), so that every trilinear footprint lies in one record.  The table
+// is dense up to kMaxDenseSlots (256 MB); beyond that, blocks of 16^3 slots
+// behind a table of 128^3 regions.  Leaves and blocks are freed once the
+// records stand.
 //
 // Record offsets are those of the 32.7 format (GridData 672 B with the map at
 // 296 and the world bbox at 560; TreeData 64 B; RootData 64 B + 32-B tiles;
@@ -43,6 +50,7 @@ template <class T> T rd(const uint8_t *p) {
 bool bit(const uint8_t *mask, uint32_t n) { return (mask[n >> 3] >> (n & 7)) & 1u; }
 
 constexpr uint64_t kMaxTop = uint64_t(1) << 24;
+constexpr uint64_t kMaxDenseSlots = uint64_t(1) << 26;
 
 struct Tables {
   int lo[3], n[3];
@@ -84,6 +92,92 @@ struct Tables {
         for (int x = t0[0]; x <= t1[0]; ++x) top[(size_t(z) * n[1] + y) * n[0] + x] = e;
   }
 };
+
+// The lookup table's extent: dense over `lo`, `n` slots, or (dense = false)
+// over regions, with `top` giving each region's block or constant
+struct TablePlan {
+  bool dense = true;
+  int lo[3] = {0, 0, 0}, n[3] = {0, 0, 0};
+  size_t entries = 0;
+  std::vector<int32_t> top, region_of_block;
+};
+
+TablePlan plan_table(const Tables &T) {
+  TablePlan p;
+  // slots that hold anything but background, and the slots below them, whose
+  // footprints reach into them
+  int64_t lo[3] = {INT64_MAX, INT64_MAX, INT64_MAX}, hi[3] = {INT64_MIN, INT64_MIN, INT64_MIN};
+  auto add = [&](int a, int64_t first, int64_t last) {
+    lo[a] = std::min(lo[a], first - 1);
+    hi[a] = std::max(hi[a], last);
+  };
+  for (int z = 0; z < T.n[2]; ++z)
+    for (int y = 0; y < T.n[1]; ++y)
+      for (int x = 0; x < T.n[0]; ++x) {
+        const int32_t t = T.top[(size_t(z) * T.n[1] + y) * T.n[0] + x];
+        if (t == -1) continue;
+        const int64_t o[3] = {16 * int64_t(T.lo[0] + x), 16 * int64_t(T.lo[1] + y),
+                              16 * int64_t(T.lo[2] + z)};
+        if (t < 0) {
+          for (int a = 0; a < 3; ++a) add(a, o[a], o[a] + 15);
+          continue;
+        }
+        const int32_t *slots = T.blocks.data() + size_t(t) * 4096;
+        for (int s = 0; s < 4096; ++s)
+          if (slots[s] != -1) {
+            const int c[3] = {s & 15, (s >> 4) & 15, s >> 8};
+            for (int a = 0; a < 3; ++a) add(a, o[a] + c[a], o[a] + c[a]);
+          }
+      }
+  if (lo[0] > hi[0]) return p;  // background everywhere
+  bool fits = true;
+  uint64_t total = 1;
+  for (int a = 0; a < 3; ++a) {
+    total *= uint64_t(hi[a] - lo[a] + 1);
+    fits = fits && total <= kMaxDenseSlots;
+    if (!fits) break;
+    p.lo[a] = int(lo[a]);
+    p.n[a] = int(hi[a] - lo[a] + 1);
+  }
+  if (fits) {
+    p.entries = size_t(total);
+    return p;
+  }
+  p.dense = false;
+  for (int a = 0; a < 3; ++a) {
+    p.lo[a] = T.lo[a] - 1;
+    p.n[a] = T.n[a] + 1;
+  }
+  p.top.resize(size_t(p.n[0]) * p.n[1] * p.n[2]);
+  auto region = [&](int x, int y, int z) {  // of `top`, by position in p's box
+    return x < 1 || y < 1 || z < 1 || x > T.n[0] || y > T.n[1] || z > T.n[2]
+               ? -1
+               : T.top[(size_t(z - 1) * T.n[1] + (y - 1)) * T.n[0] + (x - 1)];
+  };
+  for (int z = 0; z < p.n[2]; ++z)
+    for (int y = 0; y < p.n[1]; ++y)
+      for (int x = 0; x < p.n[0]; ++x) {
+        const size_t i = (size_t(z) * p.n[1] + y) * p.n[0] + x;
+        const int32_t own = region(x, y, z);
+        bool block = own >= 0;
+        for (int k = 1; k < 8 && !block; ++k)
+          block = region(x + (k & 1), y + ((k >> 1) & 1), z + (k >> 2)) != own;
+        p.top[i] = own;
+        if (block) {
+          p.top[i] = int32_t(p.region_of_block.size());
+          p.region_of_block.push_back(int32_t(i));
+        }
+      }
+  p.entries = p.region_of_block.size() * 4096;
+  return p;
+}
+
+void release(vrt_nanovdb_s *h) {
+  for (void *p : {(void *)h->top, (void *)h->consts, (void *)h->slot_ranges, (void *)h->table,
+                  (void *)h->region_top, (void *)h->recs})
+    (void)hipFree(p);
+  delete h;
+}
 
 }  // namespace
 
@@ -269,38 +363,71 @@ int vrt_nanovdb_create(vrt_context ctx, const void *grid_buffer, uint64_t bytes,
   std::vector<float> host_leaves(leaves.size() * 512);
   for (size_t i = 0; i < leaves.size(); ++i)
     std::memcpy(host_leaves.data() + 512 * i, leaves[i] + 96, 2048);
+  const TablePlan plan = plan_table(T);
+  for (int a = 0; a < 3; ++a) {
+    g.slo[a] = plan.lo[a];
+    g.sn[a] = plan.n[a];
+  }
   auto *h = new vrt_nanovdb_s(g);
+  int32_t *blocks = nullptr, *region_of_block = nullptr;
+  float *tree_leaves = nullptr;
   auto cleanup = [&](hipError_t e, const char *what) {
-    (void)hipFree(h->top);
-    (void)hipFree(h->blocks);
-    (void)hipFree(h->leaves);
-    (void)hipFree(h->consts);
-    (void)hipFree(h->slot_ranges);
-    delete h;
+    for (void *p : {(void *)blocks, (void *)region_of_block, (void *)tree_leaves})
+      (void)hipFree(p);
+    release(h);
     return hip_fail(e, what);
   };
-  const size_t nblk = T.blocks.size();
+  const size_t nblk = T.blocks.size(), nreg = plan.region_of_block.size();
   hipError_t e = hipMalloc(&h->top, T.top.size() * 4);
-  if (e == hipSuccess) e = hipMalloc(&h->blocks, std::max<size_t>(1, nblk) * 4);
-  if (e == hipSuccess) e = hipMalloc(&h->leaves, std::max<size_t>(1, host_leaves.size()) * 4);
+  if (e == hipSuccess) e = hipMalloc(&blocks, std::max<size_t>(1, nblk) * 4);
+  if (e == hipSuccess) e = hipMalloc(&tree_leaves, std::max<size_t>(1, host_leaves.size()) * 4);
   if (e == hipSuccess) e = hipMalloc(&h->consts, T.consts.size() * 4);
   if (e == hipSuccess) e = hipMalloc(&h->slot_ranges, std::max<size_t>(1, nblk) * 8);
+  // the word after the table counts its records
+  if (e == hipSuccess) e = hipMalloc(&h->table, (plan.entries + 1) * 4);
+  if (e == hipSuccess && !plan.dense) e = hipMalloc(&h->region_top, plan.top.size() * 4);
+  if (e == hipSuccess && nreg) e = hipMalloc(&region_of_block, nreg * 4);
   if (e != hipSuccess) return cleanup(e, "nanovdb allocation");
   e = hipMemcpyAsync(h->top, T.top.data(), T.top.size() * 4, hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess && nblk)
-    e = hipMemcpyAsync(h->blocks, T.blocks.data(), nblk * 4, hipMemcpyHostToDevice, ctx->stream);
+    e = hipMemcpyAsync(blocks, T.blocks.data(), nblk * 4, hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess && !host_leaves.empty())
-    e = hipMemcpyAsync(h->leaves, host_leaves.data(), host_leaves.size() * 4,
+    e = hipMemcpyAsync(tree_leaves, host_leaves.data(), host_leaves.size() * 4,
+                       hipMemcpyHostToDevice, ctx->stream);
+  if (e == hipSuccess && !plan.dense)
+    e = hipMemcpyAsync(h->region_top, plan.top.data(), plan.top.size() * 4, hipMemcpyHostToDevice,
+                       ctx->stream);
+  if (e == hipSuccess && nreg)
+    e = hipMemcpyAsync(region_of_block, plan.region_of_block.data(), nreg * 4,
                        hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess)
     e = hipMemcpyAsync(h->consts, T.consts.data(), T.consts.size() * 4, hipMemcpyHostToDevice,
                        ctx->stream);
   if (e == hipSuccess)
-    e = launch_nanovdb_slot_ranges(h->blocks, nblk, h->leaves, h->consts, h->slot_ranges,
+    e = launch_nanovdb_slot_ranges(blocks, nblk, tree_leaves, h->consts, h->slot_ranges,
                                    ctx->stream);
+  KNvTree kt{h->top, blocks, h->consts, tree_leaves, {}, {}};
+  KNvTable table{h->table, region_of_block, plan.entries, {}, {}};
+  for (int a = 0; a < 3; ++a) {
+    kt.lo[a] = T.lo[a];
+    kt.n[a] = T.n[a];
+    table.lo[a] = plan.lo[a];
+    table.n[a] = plan.n[a];
+  }
+  uint32_t *counter = reinterpret_cast<uint32_t *>(h->table + plan.entries), records = 0;
+  if (e == hipSuccess) e = hipMemsetAsync(counter, 0, 4, ctx->stream);
+  if (e == hipSuccess) e = launch_nanovdb_table(kt, table, counter, ctx->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(&records, counter, 4, hipMemcpyDeviceToHost, ctx->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+  const size_t rec_bytes = size_t(records) * VRT_BRICK_FLOATS * 4;
+  if (e == hipSuccess) e = hipMalloc(&h->recs, std::max<size_t>(4, rec_bytes));
+  if (e == hipSuccess) e = launch_nanovdb_records(kt, table, h->recs, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);  // host copies go out of scope
   if (e != hipSuccess) return cleanup(e, "nanovdb upload");
-  h->device_bytes = T.top.size() * 4 + nblk * 12 + host_leaves.size() * 4 + T.consts.size() * 4;
+  for (void *p : {(void *)blocks, (void *)region_of_block, (void *)tree_leaves}) (void)hipFree(p);
+  h->device_bytes = T.top.size() * 4 + nblk * 8 + T.consts.size() * 4 + plan.entries * 4 +
+                    plan.top.size() * 4 + rec_bytes;
   *out = h;
   return VRT_OK;
 }
@@ -327,12 +454,7 @@ int vrt_nanovdb_get_info(vrt_nanovdb g, vrt_nanovdb_info *info) {
 int vrt_nanovdb_destroy(vrt_nanovdb g) {
   if (!g) return VRT_OK;
   (void)hipSetDevice(g->device);
-  (void)hipFree(g->top);
-  (void)hipFree(g->blocks);
-  (void)hipFree(g->leaves);
-  (void)hipFree(g->consts);
-  (void)hipFree(g->slot_ranges);
-  delete g;
+  release(g);
   return VRT_OK;
 }
 

@@ -9,14 +9,16 @@
 struct vrt_nanovdb_s {
   int device = 0;
   hipStream_t stream = nullptr;  // the creating context's stream (not used after destroy)
-  // device: top table over 128^3 regions (block index >= 0, or -1 - constant),
-  // blocks of 16^3 slot entries (leaf index >= 0, or -1 - constant), leaf
-  // values (512 floats per leaf), constants (background first), per-slot
-  // value ranges of the blocks (float2)
-  int32_t *top = nullptr;
-  int32_t *blocks = nullptr;
-  float *leaves = nullptr;
+  // device, for lookups: slot table, with its region table where it is not
+  // dense, records of 9^3 voxels, constants (background first); see KVolume
+  int32_t *table = nullptr;
+  int32_t *region_top = nullptr;
+  float *recs = nullptr;
   float *consts = nullptr;
+  int slo[3] = {0, 0, 0}, sn[3] = {0, 0, 0};
+  // device, for value ranges: top table over 128^3 regions (block index >= 0,
+  // or -1 - constant), per-slot value ranges of the blocks (float2)
+  int32_t *top = nullptr;
   float *slot_ranges = nullptr;
   int lo[3] = {0, 0, 0}, n[3] = {0, 0, 0};  // top-table origin (in 128-voxel units) / dims
   uint64_t block_count = 0;

@@ -102,12 +102,16 @@ int make_nanovdb_volume(const vrt_volume &in, int lds_offset, KVolume &v) {
   v.glo = v.blo;
   v.ghi = v.bhi;
   v.cell_size = 1.f;
-  v.leaves = g->leaves;
+  v.nv_recs = g->recs;
+  v.nv_tab = g->table;
+  v.nv_rtop = g->region_top;
+  v.nv_bg = g->background;
   v.nv_top = g->top;
-  v.nv_blocks = g->blocks;
   v.nv_consts = g->consts;
   v.nv_slot_ranges = g->slot_ranges;
   for (int a = 0; a < 3; ++a) {
+    v.nv_slo[a] = g->slo[a];
+    v.nv_sn[a] = g->sn[a];
     v.nv_lo[a] = g->lo[a];
     v.nv_n[a] = g->n[a];
     v.nv_vec[a] = g->vec_f[a];

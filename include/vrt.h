@@ -356,10 +356,10 @@ typedef struct vrt_nanovdb_info {
   int top_origin[3];                /* index of top entry (0,0,0) / 128 */
   int top_dims[3];                  /* top table dims */
   uint64_t blocks;                  /* lower nodes inside the bounds */
-  uint64_t leaves;                  /* leaves copied to the device */
+  uint64_t leaves;                  /* leaves inside the bounds */
   uint64_t constants;               /* distinct constants (background first) */
   uint64_t active_voxels;           /* TreeData::mVoxelCount */
-  uint64_t device_bytes;            /* tables + leaves + constants + slot ranges */
+  uint64_t device_bytes;            /* tables + records + constants + slot ranges */
 } vrt_nanovdb_info;
 
 VRT_API int vrt_nanovdb_create(vrt_context ctx, const void *grid_buffer, uint64_t bytes,
