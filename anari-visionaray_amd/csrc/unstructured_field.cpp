@@ -10,6 +10,7 @@
 #include <thread>
 #include <vector>
 
+#include "render_kernels.h"
 #include "tet_grid.h"
 #include "unstructured_internal.h"
 #include "vrt.h"
@@ -141,6 +142,7 @@ int vrt_unstructured_create(vrt_context ctx, const float *pos, const float *vdat
   auto cleanup = [&](hipError_t e, const char *what) {
     (void)hipFree(h->start);
     (void)hipFree(h->recs);
+    (void)hipFree(h->planes);
     (void)hipFree(h->rec_cell);
     (void)hipFree(h->tets);
     delete h;
@@ -155,6 +157,7 @@ int vrt_unstructured_create(vrt_context ctx, const float *pos, const float *vdat
                cell_bytes = rec_cell.size() * 4, tet_bytes = tets.size() * sizeof(float4);
   hipError_t e = hipMalloc(&h->start, start_bytes);
   if (e == hipSuccess) e = hipMalloc(&h->recs, std::max<size_t>(rec_bytes, 64));
+  if (e == hipSuccess) e = hipMalloc(&h->planes, std::max<size_t>(rec_bytes / 2, 64));
   if (e == hipSuccess) e = hipMalloc(&h->rec_cell, std::max<size_t>(cell_bytes, 4));
   if (e == hipSuccess) e = hipMalloc(&h->tets, tet_bytes);
   if (e != hipSuccess) return cleanup(e, "unstructured field allocation");
@@ -166,9 +169,11 @@ int vrt_unstructured_create(vrt_context ctx, const float *pos, const float *vdat
                        ctx->stream);
   if (e == hipSuccess)
     e = hipMemcpyAsync(h->tets, tets.data(), tet_bytes, hipMemcpyHostToDevice, ctx->stream);
+  if (e == hipSuccess)
+    e = launch_tet_planes(h->start, h->recs, h->lo, h->inv_cell, h->dims, h->planes, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);  // host copies go out of scope
   if (e != hipSuccess) return cleanup(e, "unstructured field upload");
-  h->device_bytes = start_bytes + rec_bytes + cell_bytes + tet_bytes;
+  h->device_bytes = start_bytes + rec_bytes + rec_bytes / 2 + cell_bytes + tet_bytes;
   *out = h;
   return VRT_OK;
 }
@@ -199,6 +204,7 @@ int vrt_unstructured_destroy(vrt_unstructured f) {
   (void)hipSetDevice(f->device);
   (void)hipFree(f->start);
   (void)hipFree(f->recs);
+  (void)hipFree(f->planes);
   (void)hipFree(f->rec_cell);
   (void)hipFree(f->tets);
   delete f;

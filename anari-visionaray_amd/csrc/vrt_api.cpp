@@ -137,6 +137,7 @@ int make_unstructured_volume(const vrt_volume &in, int lds_offset, KVolume &v) {
   v.cell_size = f->cell_size;
   v.ug_start = f->start;
   v.ug_recs = f->recs;
+  v.ug_planes = f->planes;
   v.ug_cell = f->rec_cell;
   v.ug_tets = f->tets;
   v.ug_num_tets = uint32_t(f->num_tets);
