@@ -80,13 +80,16 @@ struct Builder {
       nodes[id].count = count;
       return id;
     };
-    if (count <= 4 || level >= 60) return make_leaf();
+    // below level 60 (a sweep that peels off a few triangles per level) lists
+    // are halved; the traversal holds a leaf's count in a byte
+    const bool halve = level >= 60;
+    if (count <= 4 || (halve && count <= 255)) return make_leaf();
     int axis = 0;
     for (int a = 1; a < 3; ++a)
       if (cbox.hi[a] - cbox.lo[a] > cbox.hi[axis] - cbox.lo[axis]) axis = a;
     const float ext = cbox.hi[axis] - cbox.lo[axis];
     int mid = -1;
-    if (ext > 0.f) {
+    if (ext > 0.f && !halve) {
       constexpr int kBins = 16;
       Box bb[kBins];
       int bn[kBins] = {0};
