@@ -2519,13 +2519,20 @@ __global__ void __launch_bounds__(256, 3)
   auto band = [&](int i) {
     return ((nch + kQueues - 1 - uint32_t(i)) / kQueues) << (2 * kChunkLog2);
   };
+  // Pixels a wave holds at a time and claims at once: 64, or where the frame
+  // has fewer than 64 per wave the power of two (at least 8) that gives every
+  // wave some.  A pass lasts as long as its longest ray, and a frame that
+  // leaves waves idle as long as its longest path, so fewer lanes a wave end
+  // it sooner: 200x150 pixels (16 a wave) 300 -> 247 us.
+  uint32_t step = 64u;
+  while (step > 8u && nch * (1u << (2 * kChunkLog2 - 3)) <= (step / 16u) * gridDim.x * 4u) step /= 2u;
   // the grid is a multiple of 8 workgroups: `waves` of them start on each
-  // queue, each with the 64 pixels of its position
+  // queue, each with the pixels of its position
   const uint32_t waves = gridDim.x / kQueues * 4u;
   // wave-uniform local pool
-  uint32_t pool_base = 64u * ((blockIdx.x / kQueues) * 4u +
-                              uint32_t(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)));
-  uint32_t pool_left = pool_base < band(q) ? 64u : 0u;
+  uint32_t pool_base = step * ((blockIdx.x / kQueues) * 4u +
+                               uint32_t(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)));
+  uint32_t pool_left = pool_base < band(q) ? step : 0u;
   bool drained = false;
   int px = 0, py = 0;
 
@@ -2537,17 +2544,18 @@ __global__ void __launch_bounds__(256, 3)
     const bool chained = __ballot(chain) != 0ull;
     // ---- refill idle lanes ----------------------------------------------------
     unsigned long long idle = chained ? 0ull : __ballot(st.pixel < 0);
-    if (P.refill_min > 1 && __popcll(idle) < P.refill_min && __ballot(st.pixel >= 0) != 0ull)
-      idle = 0ull;  // refill later, for more lanes at once
-    while (idle && !drained) {
+    // lanes to refill: idle ones up to `step` pixels in the wave
+    uint32_t room = step - min(step, uint32_t(__popcll(~idle)));
+    if (P.refill_min > 1 && room < uint32_t(P.refill_min) && ~idle != 0ull)
+      room = 0u;  // refill later, for more lanes at once
+    while (idle && room && !drained) {
       if (pool_left == 0) {
-        pool_base = queue_claim(queues, q, 64u, 64u * waves, band);
+        pool_base = queue_claim(queues, q, step, step * waves, band);
         drained = pool_base == kDrained;
         if (drained) break;
-        pool_left = 64u;  // (a band is a multiple of 64)
+        pool_left = step;  // (a band is a multiple of 64)
       }
-      const uint32_t nidle = uint32_t(__popcll(idle));
-      const uint32_t take = min(nidle, pool_left);
+      const uint32_t take = min(room, pool_left);
       const uint32_t rank = uint32_t(__popcll(idle & below));
       chunk_pixel(q, pool_base + rank, nchx, px, py);
       if (st.pixel < 0 && rank < take && px < W && py < H) {
@@ -2563,8 +2571,8 @@ __global__ void __launch_bounds__(256, 3)
       }
       pool_base += take;
       pool_left -= take;
+      room -= take;
       idle = __ballot(st.pixel < 0);
-      if (take == nidle) break;  // every idle lane was offered a pixel
     }
     if (!chained && __ballot(st.pixel >= 0) == 0ull) {
       // no lane holds a pixel: either every queue is drained, or the last
