@@ -2178,7 +2178,8 @@ __device__ inline void taa_vertex(const KFrame &F, const KParams &P, const PathS
 // on.
 template <bool NRC, bool AREA, int FIELD, bool GRAD>
 __device__ inline bool path_shade(PathState &st, const KScene &sc, const KParams &P,
-                                  const KNrc &N, const KFrame &F, const PassHit &h) {
+                                  const KNrc &N, const KFrame &F, const PassHit &h,
+                                  uint32_t &v2_paths) {
   KRay ray;
   ray.ori = st.ori;
   ray.dir = st.dir;
@@ -2193,7 +2194,7 @@ __device__ inline bool path_shade(PathState &st, const KScene &sc, const KParams
   }
   if constexpr (NRC) {
     const bool v2 = st.rayType == Radiance && h.kind == kVolume && st.bounceID == N.qbounce;
-    (void)wave_claim(&N.ctr[2], v2);  // vertex-2 paths of this frame
+    v2_paths += v2 ? 1u : 0u;
     const bool want_train = v2 && st.train_sel;
     const uint32_t tslot = wave_claim(&N.ctr[1], want_train);
     const bool is_train = want_train && tslot < uint32_t(N.t_cap);
@@ -2514,6 +2515,7 @@ __global__ void __launch_bounds__(256, 3)
   PathState st;
   st.pixel = -1;
   uint32_t lookups = 0, hit_samples = 0;
+  uint32_t v2_paths = 0;  // radiance cache: paths that reached the query vertex
   int q = int(blockIdx.x) & (kQueues - 1);  // wave-uniform queue
   // pixels of queue i: the chunks c = i, i+8, ... times 1024 pixels
   auto band = [&](int i) {
@@ -2525,6 +2527,12 @@ __global__ void __launch_bounds__(256, 3)
   // leaves waves idle as long as its longest path, so fewer lanes a wave end
   // it sooner: 200x150 pixels (16 a wave) 300 -> 247 us.
   uint32_t step = 64u;
+  // Later claims: 16 pixels where a pass is long (surfaces, tetrahedra, a
+  // NanoVDB walk), so that the frame's last pixels go to whichever waves are
+  // free (claims of 64 / 16: mixed surfaces and volume 5.50 / 5.17 ms,
+  // tetrahedra 2.77 / 2.66, cloud 5.69 / 5.43); 64 where passes are short and
+  // the claim's round trip shows (fBm 0.82 / 0.87 ms, cache frames 2.63 / 2.78)
+  constexpr uint32_t kMaxClaim = !NRC && (AREA || FIELD != kStructuredField) ? 16u : 64u;
   while (step > 8u && nch * (1u << (2 * kChunkLog2 - 3)) <= (step / 16u) * gridDim.x * 4u) step /= 2u;
   // the grid is a multiple of 8 workgroups: `waves` of them start on each
   // queue, each with the pixels of its position
@@ -2550,10 +2558,11 @@ __global__ void __launch_bounds__(256, 3)
       room = 0u;  // refill later, for more lanes at once
     while (idle && room && !drained) {
       if (pool_left == 0) {
-        pool_base = queue_claim(queues, q, step, step * waves, band);
+        const uint32_t claim = min(step, kMaxClaim);
+        pool_base = queue_claim(queues, q, claim, step * waves, band);
         drained = pool_base == kDrained;
         if (drained) break;
-        pool_left = step;  // (a band is a multiple of 64)
+        pool_left = claim;  // (a band is a multiple of 64)
       }
       const uint32_t take = min(room, pool_left);
       const uint32_t rank = uint32_t(__popcll(idle & below));
@@ -2594,7 +2603,7 @@ __global__ void __launch_bounds__(256, 3)
       const PassHit hit = intersect_all<AREA, FIELD, INST>(sc, ray, shadow, st.bounceID, s_tf, steps,
                                                     st.srng, lookups, bstack, lnodes,
                                                     shadow && P.ratio_tracking != 0);
-      if (path_shade<NRC, AREA, FIELD, GRAD>(st, sc, P, N, F, hit)) {
+      if (path_shade<NRC, AREA, FIELD, GRAD>(st, sc, P, N, F, hit, v2_paths)) {
         float4 color = P.bg;
         if (st.firstHit) color = make_float4(st.intensity.x, st.intensity.y, st.intensity.z, 1.f);
         hit_samples += st.firstHit ? 1u : 0u;
@@ -2647,6 +2656,12 @@ __global__ void __launch_bounds__(256, 3)
         chain = P.chain_passes && st.rayType != Radiance;
       }
     }
+  }
+  if constexpr (NRC) {
+    // counted once per wave: an atomic per pass on the counters' line would
+    // wait for every other wave's
+    for (int o = 32; o > 0; o >>= 1) v2_paths += __shfl_xor(v2_paths, o, 64);
+    if (lane == 0u && v2_paths) atomicAdd(&N.ctr[2], v2_paths);
   }
   if (F.counters) {
     wave_add_counter(&F.counters[0], lookups);
