@@ -815,13 +815,20 @@ __device__ inline bool bvh_hit(const KSurface &S, const KRay &r, bool any, float
         node = -2;  // pop once the leaves are tested
       }
     } while (counts == 0u && node >= 0 && __popcll(__ballot(true)) * kWalkShare >= lanes0);
-    // the leaves' triangles, in one loop for all four children
-    while (counts != 0u) {
-      const int c = (__ffs(int(counts)) - 1) >> 3;
-      const int q0 = c == 0 ? leaf[0] : c == 1 ? leaf[1] : c == 2 ? leaf[2] : leaf[3];
-      const uint32_t k = ((counts >> (8 * c)) & 255u) - 1u;
-      counts -= 1u << (8 * c);
-      const float4 *q = S.tris + 3 * (size_t(q0) + k);
+    // the leaves' triangles, in one loop for all four children, each leaf's in
+    // ascending order (any-hit calls return the first one met)
+    uint32_t q0 = 0;
+    uint32_t left = 0;
+    while ((counts | left) != 0u) {
+      if (left == 0u) {
+        const int c = (__ffs(int(counts)) - 1) >> 3;
+        q0 = uint32_t(c == 0 ? leaf[0] : c == 1 ? leaf[1] : c == 2 ? leaf[2] : leaf[3]);
+        left = (counts >> (8 * c)) & 255u;
+        counts &= ~(255u << (8 * c));
+      }
+      const uint32_t k = q0++;
+      --left;
+      const float4 *q = S.tris + 3 * size_t(k);
       const float4 a = q[0], b = q[1], d = q[2];
       float t, u, v;
       if (!tri_test(r, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), mk(d.x, d.y, d.z), t, u, v))
@@ -831,7 +838,7 @@ __device__ inline bool bvh_hit(const KSurface &S, const KRay &r, bool any, float
       found = true;
       tbest = t;
       prim = p;
-      rec = uint32_t(q0) + k;
+      rec = k;
       if (any) return true;
     }
     // unless a closer triangle was found since

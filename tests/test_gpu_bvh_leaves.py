@@ -47,3 +47,33 @@ def test_long_lists_below_level_60(pkg, oracle, gpu_ctx, tail):
     ta, pa = vrt.intersect_surfaces(gpu_ctx, scene, r, True)
     np.testing.assert_array_equal(pa >= 0, po >= 0)
     assert (po >= 0).mean() > 0.05
+
+
+@pytest.mark.parametrize("count", [1, 2, 3, 4])
+def test_any_hit_returns_the_first_of_a_leaf(pkg, gpu_ctx, count):
+    """Up to 4 triangles are one leaf, held in the order given: an any-hit
+    call returns the first that the ray meets, whatever lies nearer."""
+    vrt = pkg.vrt
+    tri = np.zeros((count, 3, 3), np.float32)
+    for i in range(count):  # planes z = -i; the first ones also narrower in x
+        tri[i] = [(-2 - i, -2, -i), (2 + i, -2, -i), (0, 4 + 2 * i, -i)]
+    mesh = vrt.DeviceMesh(gpu_ctx, tri.reshape(-1, 3), None, "sah")  # (outlives the scene)
+    scene = vrt.make_scene([], [], [(mesh, (0.7, 0.7, 0.7))])
+    rng = np.random.default_rng(count)
+    r = np.zeros((4000, 8), np.float32)
+    r[:, :3] = rng.uniform(-5, 5, (4000, 3))
+    r[:, 2] = np.where(np.arange(4000) % 2, 3.0, -7.0)
+    r[:, 5] = np.where(np.arange(4000) % 2, -1.0, 1.0)
+    r[:, 7] = 1e30
+    hit = np.stack([(r[:, 1] > -2) & (r[:, 1] < (4 + 2 * i) - (6 + 2 * i) * np.abs(r[:, 0]) / (2 + i))
+                    for i in range(count)])
+    # (edges: no ray within 1e-3 of one)
+    edge = np.stack([np.minimum(np.abs(r[:, 1] + 2), np.abs(
+        (4 + 2 * i) - (6 + 2 * i) * np.abs(r[:, 0]) / (2 + i) - r[:, 1])) for i in range(count)])
+    keep = edge.min(0) > 1e-3
+    first = np.where(hit.any(0), hit.argmax(0), -1)
+    t, p = vrt.intersect_surfaces(gpu_ctx, scene, r, True)
+    np.testing.assert_array_equal(p[keep], first[keep])
+    got = keep & (first >= 0)
+    np.testing.assert_allclose(t[got], np.abs(r[got, 2] + first[got]), rtol=1e-5)
+    assert got.sum() > 300
