@@ -32,6 +32,23 @@ __host__ __device__ inline float max3(f3 a) { return fmaxf(a.x, fmaxf(a.y, a.z))
 __host__ __device__ inline f3 fabs3(f3 a) { return {fabsf(a.x), fabsf(a.y), fabsf(a.z)}; }
 __host__ __device__ inline float comp(f3 a, int i) { return i == 0 ? a.x : (i == 1 ? a.y : a.z); }
 
+// A NanoVDB tree as two tables (see nanovdb_field.cpp): top table over 128^3
+// regions (>= 0 block index, else -1 - constant) of origin lo (in 128-voxel
+// units) and dims n; blocks of 16^3 slot entries (>= 0 leaf, else -1 -
+// constant); leaf values (512 each; null once the records hold all that
+// lookups read); value range of each slot of the blocks.  In device memory:
+// the kernels' arguments hold its address only, as few lookups read it and
+// each word of a volume costs the renderers registers.
+struct KNvTree {
+  const int32_t *top, *blocks;
+  const float *consts, *leaves;
+  const float2 *slot_ranges;
+  int lo[3], n[3];
+};
+
+// entry of a nanovdb lookup table whose voxels are read from the tree tables
+constexpr int32_t kNvTreeEntry = INT32_MIN;
+
 // One volume instance, derived from vrt_volume on the host.
 struct KVolume {
   int field_type;
@@ -59,23 +76,17 @@ struct KVolume {
   f3 glo, ghi;         // majorant grid bounds in voxel space
   // nanovdb lookups: a table over the 8^3-voxel slots [nv_slo, nv_slo +
   // nv_sn) whose entry is a record of 9^3 voxels in nv_recs (>= 0,
-  // VRT_BRICK_FLOATS each) or -1 - index into nv_consts (0: the background,
-  // also outside); with nv_rtop the table holds blocks of 16^3 slots, nv_slo
-  // and nv_sn count 128^3 regions and nv_rtop gives a region's block or
-  // constant.  World -> index map, filter
+  // VRT_BRICK_FLOATS each), kNvTreeEntry or -1 - index into the tree's constants
+  // (0: the background, also outside); with nv_rtop the table holds blocks of 16^3
+  // slots, nv_slo and nv_sn count 128^3 regions and nv_rtop gives a region's
+  // block, kNvTreeEntry or constant.  World -> index map, filter
   const float *nv_recs;
   const int32_t *nv_tab;
   const int32_t *nv_rtop;
-  const float *nv_consts;
+  const KNvTree *nv_tree;
   float nv_bg;
   int nv_slo[3], nv_sn[3];
   float nv_inv[9], nv_vec[3];
-  // nanovdb value ranges: top table over 128^3 regions (>= 0 block index,
-  // else a constant), value range of each slot of the blocks, top origin (in
-  // 128-voxel units) / dims
-  const int32_t *nv_top;
-  const float *nv_slot_ranges;
-  int nv_lo[3], nv_n[3];
   int filter;
   // unstructured: point-location grid (list start per grid cell, dims
   // product + 1 entries; tetrahedron copies of four float4 {x, y, z, value}

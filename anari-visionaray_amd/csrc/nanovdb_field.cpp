@@ -13,14 +13,25 @@
 //    (i&7)<<6 | (j&7)<<3 | (k&7).
 // Grids with huge tiles stay small because a tile costs one top entry.
 //
-// From these the GPU builds what lookups read: a table with one entry per
-// 8^3 slot of the box that holds anything but background, and, for each slot
-// whose 9^3 voxels (its own and the first layers of its 7 upper neighbours)
-// are not one constant, a record of these voxels (VRT_BRICK_FLOATS floats, x
-// fastest), so that every trilinear footprint lies in one record.  The table
-// is dense up to kMaxDenseSlots (256 MB); beyond that, blocks of 16^3 slots
-// behind a table of 128^3 regions.  Leaves and blocks are freed once the
-// records stand.
+// From these the GPU builds what lookups read: a table with one entry per 8^3
+// slot of the box that holds anything but background.  A trilinear footprint
+// that starts in a slot reads its 9^3 voxels (its own and the first layers of
+// its 7 upper neighbours), so the entry is
+//  * where one of these 8 slots holds a leaf: a record of the 9^3 voxels
+//    (VRT_BRICK_FLOATS floats, x fastest), so that the footprint lies in it;
+//  * else, where they hold one constant: -1 - c;
+//  * else (borders between tiles): kNvTreeEntry, whose taps walk the tables above.
+// The table is dense where that takes no more than the tables above (or 16
+// MB, and at most 256 MB); else it has blocks of 16^3 slots behind a table of
+// 128^3 regions, whose entry is a block where the region or one of its 7 upper
+// neighbours holds a lower node, else their constant or kNvTreeEntry.
+//
+// Records take 1.4 times the leaves' memory for a solid field, up to 11.5
+// times for leaves that touch no other (8 records of 2,944 B each).  Where they would
+// take more than 64 MB and more than 8 times the tree's tables, or half of the
+// device's free memory, no records are made: every such slot is kNvTreeEntry, a
+// lookup costs what the tree's three dependent reads cost, and the leaves
+// stay.  Else they are freed once the records stand.
 //
 // Record offsets are those of the 32.7 format (GridData 672 B with the map at
 // 296 and the world bbox at 560; TreeData 64 B; RootData 64 B + 32-B tiles;
@@ -50,7 +61,9 @@ template <class T> T rd(const uint8_t *p) {
 bool bit(const uint8_t *mask, uint32_t n) { return (mask[n >> 3] >> (n & 7)) & 1u; }
 
 constexpr uint64_t kMaxTop = uint64_t(1) << 24;
+constexpr uint64_t kMinDenseSlots = uint64_t(1) << 22;
 constexpr uint64_t kMaxDenseSlots = uint64_t(1) << 26;
+constexpr uint64_t kSmallRecords = uint64_t(64) << 20;  // bytes
 
 struct Tables {
   int lo[3], n[3];
@@ -94,15 +107,25 @@ struct Tables {
 };
 
 // The lookup table's extent: dense over `lo`, `n` slots, or (dense = false)
-// over regions, with `top` giving each region's block or constant
+// over regions, with `top` giving each region's block, kNvTreeEntry or constant
 struct TablePlan {
   bool dense = true;
   int lo[3] = {0, 0, 0}, n[3] = {0, 0, 0};
   size_t entries = 0;
   std::vector<int32_t> top, region_of_block;
+  bool reads_leaves = false;  // regions' kNvTreeEntry entries reach into blocks
 };
 
-TablePlan plan_table(const Tables &T) {
+// whether `bytes` more for lookups are in proportion to the tree's own tables
+// and leave as much of the device's memory as they take
+bool worth_memory(uint64_t bytes, uint64_t tree_bytes) {
+  if (bytes <= kSmallRecords) return true;
+  size_t free_bytes = 0, total = 0;
+  return bytes <= 8 * tree_bytes && hipMemGetInfo(&free_bytes, &total) == hipSuccess &&
+         bytes <= free_bytes / 2;
+}
+
+TablePlan plan_table(const Tables &T, uint64_t tree_bytes) {
   TablePlan p;
   // slots that hold anything but background, and the slots below them, whose
   // footprints reach into them
@@ -130,16 +153,17 @@ TablePlan plan_table(const Tables &T) {
           }
       }
   if (lo[0] > hi[0]) return p;  // background everywhere
+  const uint64_t limit = std::min(kMaxDenseSlots, std::max(kMinDenseSlots, tree_bytes / 4));
   bool fits = true;
   uint64_t total = 1;
   for (int a = 0; a < 3; ++a) {
     total *= uint64_t(hi[a] - lo[a] + 1);
-    fits = fits && total <= kMaxDenseSlots;
+    fits = fits && total <= limit;
     if (!fits) break;
     p.lo[a] = int(lo[a]);
     p.n[a] = int(hi[a] - lo[a] + 1);
   }
-  if (fits) {
+  if (fits && worth_memory(4 * total, tree_bytes)) {
     p.entries = size_t(total);
     return p;
   }
@@ -154,30 +178,52 @@ TablePlan plan_table(const Tables &T) {
                ? -1
                : T.top[(size_t(z - 1) * T.n[1] + (y - 1)) * T.n[0] + (x - 1)];
   };
-  for (int z = 0; z < p.n[2]; ++z)
-    for (int y = 0; y < p.n[1]; ++y)
-      for (int x = 0; x < p.n[0]; ++x) {
-        const size_t i = (size_t(z) * p.n[1] + y) * p.n[0] + x;
-        const int32_t own = region(x, y, z);
-        bool block = own >= 0;
-        for (int k = 1; k < 8 && !block; ++k)
-          block = region(x + (k & 1), y + ((k >> 1) & 1), z + (k >> 2)) != own;
-        p.top[i] = own;
-        if (block) {
-          p.top[i] = int32_t(p.region_of_block.size());
-          p.region_of_block.push_back(int32_t(i));
+  // blocks for the regions that hold a lower node, and for those below them
+  // if these (up to 7 each) are worth their memory
+  size_t wide = 0;
+  for (int pass = 0; pass < 2; ++pass) {
+    const bool below = pass == 0 || worth_memory(wide * 16384, tree_bytes);
+    for (int z = 0; z < p.n[2]; ++z)
+      for (int y = 0; y < p.n[1]; ++y)
+        for (int x = 0; x < p.n[0]; ++x) {
+          const size_t i = (size_t(z) * p.n[1] + y) * p.n[0] + x;
+          const int32_t own = region(x, y, z);
+          bool node = own >= 0, differ = false;
+          for (int k = 1; k < 8; ++k) {
+            const int32_t r = region(x + (k & 1), y + ((k >> 1) & 1), z + (k >> 2));
+            node = node || r >= 0;
+            differ = differ || r != own;
+          }
+          const bool block = own >= 0 || (node && below);
+          if (pass == 0) {
+            wide += block ? 1 : 0;
+          } else if (block) {
+            p.top[i] = int32_t(p.region_of_block.size());
+            p.region_of_block.push_back(int32_t(i));
+          } else {
+            p.top[i] = differ ? kNvTreeEntry : own;
+            p.reads_leaves = p.reads_leaves || node;
+          }
         }
-      }
+  }
   p.entries = p.region_of_block.size() * 4096;
   return p;
 }
 
 void release(vrt_nanovdb_s *h) {
-  for (void *p : {(void *)h->top, (void *)h->consts, (void *)h->slot_ranges, (void *)h->table,
-                  (void *)h->region_top, (void *)h->recs})
-    (void)hipFree(p);
+  for (void *p : {(void *)h->mem, (void *)h->leaves, (void *)h->recs}) (void)hipFree(p);
   delete h;
 }
+
+// the parts of the tables' allocation, each aligned to 256 B
+struct Parts {
+  size_t bytes = 0;
+  size_t add(size_t n) {
+    const size_t at = bytes;
+    bytes += (n + 255) / 256 * 256;
+    return at;
+  }
+};
 
 }  // namespace
 
@@ -363,71 +409,90 @@ int vrt_nanovdb_create(vrt_context ctx, const void *grid_buffer, uint64_t bytes,
   std::vector<float> host_leaves(leaves.size() * 512);
   for (size_t i = 0; i < leaves.size(); ++i)
     std::memcpy(host_leaves.data() + 512 * i, leaves[i] + 96, 2048);
-  const TablePlan plan = plan_table(T);
+  const size_t nblk = T.blocks.size(), leaf_bytes = host_leaves.size() * 4;
+  const uint64_t tree_bytes = T.top.size() * 4 + nblk * 4 + leaf_bytes;
+  const TablePlan plan = plan_table(T, tree_bytes);
   for (int a = 0; a < 3; ++a) {
     g.slo[a] = plan.lo[a];
     g.sn[a] = plan.n[a];
   }
+  // One allocation: what the host made, in one copy, then what the GPU makes.
+  // (A creation is a chain of round trips: an allocation and a copy for each
+  // array took 0.04 ms longer.)
+  KNvTree kt{};
+  const uint32_t zero = 0;  // the count of records
+  struct {
+    const void *src;
+    size_t bytes, at;
+  } up[] = {{&kt, sizeof kt, 0},
+            {T.top.data(), T.top.size() * 4, 0},
+            {T.consts.data(), T.consts.size() * 4, 0},
+            {T.blocks.data(), nblk * 4, 0},
+            {plan.top.data(), plan.top.size() * 4, 0},
+            {plan.region_of_block.data(), plan.region_of_block.size() * 4, 0},
+            {&zero, sizeof zero, 0}};
+  Parts P;
+  for (auto &u : up) u.at = P.add(u.bytes);
+  const size_t stage_bytes = P.bytes;
+  const size_t ranges_at = P.add(nblk * 8), table_at = P.add(plan.entries * 4);
+
   auto *h = new vrt_nanovdb_s(g);
-  int32_t *blocks = nullptr, *region_of_block = nullptr;
-  float *tree_leaves = nullptr;
   auto cleanup = [&](hipError_t e, const char *what) {
-    for (void *p : {(void *)blocks, (void *)region_of_block, (void *)tree_leaves})
-      (void)hipFree(p);
     release(h);
     return hip_fail(e, what);
   };
-  const size_t nblk = T.blocks.size(), nreg = plan.region_of_block.size();
-  hipError_t e = hipMalloc(&h->top, T.top.size() * 4);
-  if (e == hipSuccess) e = hipMalloc(&blocks, std::max<size_t>(1, nblk) * 4);
-  if (e == hipSuccess) e = hipMalloc(&tree_leaves, std::max<size_t>(1, host_leaves.size()) * 4);
-  if (e == hipSuccess) e = hipMalloc(&h->consts, T.consts.size() * 4);
-  if (e == hipSuccess) e = hipMalloc(&h->slot_ranges, std::max<size_t>(1, nblk) * 8);
-  // the word after the table counts its records
-  if (e == hipSuccess) e = hipMalloc(&h->table, (plan.entries + 1) * 4);
-  if (e == hipSuccess && !plan.dense) e = hipMalloc(&h->region_top, plan.top.size() * 4);
-  if (e == hipSuccess && nreg) e = hipMalloc(&region_of_block, nreg * 4);
+  hipError_t e = hipMalloc(&h->mem, P.bytes);
+  if (e == hipSuccess && leaf_bytes) e = hipMalloc(&h->leaves, leaf_bytes);
   if (e != hipSuccess) return cleanup(e, "nanovdb allocation");
-  e = hipMemcpyAsync(h->top, T.top.data(), T.top.size() * 4, hipMemcpyHostToDevice, ctx->stream);
-  if (e == hipSuccess && nblk)
-    e = hipMemcpyAsync(blocks, T.blocks.data(), nblk * 4, hipMemcpyHostToDevice, ctx->stream);
-  if (e == hipSuccess && !host_leaves.empty())
-    e = hipMemcpyAsync(tree_leaves, host_leaves.data(), host_leaves.size() * 4,
-                       hipMemcpyHostToDevice, ctx->stream);
-  if (e == hipSuccess && !plan.dense)
-    e = hipMemcpyAsync(h->region_top, plan.top.data(), plan.top.size() * 4, hipMemcpyHostToDevice,
-                       ctx->stream);
-  if (e == hipSuccess && nreg)
-    e = hipMemcpyAsync(region_of_block, plan.region_of_block.data(), nreg * 4,
-                       hipMemcpyHostToDevice, ctx->stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(h->consts, T.consts.data(), T.consts.size() * 4, hipMemcpyHostToDevice,
-                       ctx->stream);
-  if (e == hipSuccess)
-    e = launch_nanovdb_slot_ranges(blocks, nblk, tree_leaves, h->consts, h->slot_ranges,
-                                   ctx->stream);
-  KNvTree kt{h->top, blocks, h->consts, tree_leaves, {}, {}};
-  KNvTable table{h->table, region_of_block, plan.entries, {}, {}};
+  auto ints = [&](size_t at) { return reinterpret_cast<int32_t *>(h->mem + at); };
+  h->tree = reinterpret_cast<const KNvTree *>(h->mem + up[0].at);
+  if (!plan.dense) h->region_top = ints(up[4].at);
+  h->table = ints(table_at);
+  float *slot_ranges = reinterpret_cast<float *>(h->mem + ranges_at);
+  uint32_t *counter = reinterpret_cast<uint32_t *>(h->mem + up[6].at), records = 0;
+  kt.top = ints(up[1].at);
+  kt.blocks = ints(up[3].at);
+  kt.consts = reinterpret_cast<const float *>(h->mem + up[2].at);
+  kt.leaves = h->leaves;
+  kt.slot_ranges = reinterpret_cast<const float2 *>(slot_ranges);
+  KNvTable table{h->table, plan.dense ? nullptr : ints(up[5].at), plan.entries, {}, {}};
   for (int a = 0; a < 3; ++a) {
     kt.lo[a] = T.lo[a];
     kt.n[a] = T.n[a];
     table.lo[a] = plan.lo[a];
     table.n[a] = plan.n[a];
   }
-  uint32_t *counter = reinterpret_cast<uint32_t *>(h->table + plan.entries), records = 0;
-  if (e == hipSuccess) e = hipMemsetAsync(counter, 0, 4, ctx->stream);
-  if (e == hipSuccess) e = launch_nanovdb_table(kt, table, counter, ctx->stream);
+  std::vector<char> stage(stage_bytes);
+  for (const auto &u : up)
+    if (u.bytes) std::memcpy(stage.data() + u.at, u.src, u.bytes);
+  e = hipMemcpyAsync(h->mem, stage.data(), stage_bytes, hipMemcpyHostToDevice, ctx->stream);
+  if (e == hipSuccess && leaf_bytes)
+    e = hipMemcpyAsync(h->leaves, host_leaves.data(), leaf_bytes, hipMemcpyHostToDevice,
+                       ctx->stream);
+  if (e == hipSuccess)
+    e = launch_nanovdb_slot_ranges(kt.blocks, nblk, kt.leaves, kt.consts, slot_ranges,
+                                   ctx->stream);
+  if (e == hipSuccess) e = launch_nanovdb_table(kt, table, true, counter, ctx->stream);
   if (e == hipSuccess)
     e = hipMemcpyAsync(&records, counter, 4, hipMemcpyDeviceToHost, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  const size_t rec_bytes = size_t(records) * VRT_BRICK_FLOATS * 4;
-  if (e == hipSuccess) e = hipMalloc(&h->recs, std::max<size_t>(4, rec_bytes));
-  if (e == hipSuccess) e = launch_nanovdb_records(kt, table, h->recs, ctx->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);  // host copies go out of scope
+  size_t rec_bytes = size_t(records) * VRT_BRICK_FLOATS * 4;
+  bool keep_leaves = plan.reads_leaves;
+  if (e == hipSuccess && records && !worth_memory(rec_bytes, tree_bytes)) {
+    rec_bytes = 0;
+    keep_leaves = true;
+    e = launch_nanovdb_table(kt, table, false, counter, ctx->stream);
+  } else if (e == hipSuccess && records) {
+    e = hipMalloc(&h->recs, rec_bytes);
+    if (e == hipSuccess) e = launch_nanovdb_records(kt, table, h->recs, ctx->stream);
+  }
+  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);  // (usable on every stream)
   if (e != hipSuccess) return cleanup(e, "nanovdb upload");
-  for (void *p : {(void *)blocks, (void *)region_of_block, (void *)tree_leaves}) (void)hipFree(p);
-  h->device_bytes = T.top.size() * 4 + nblk * 8 + T.consts.size() * 4 + plan.entries * 4 +
-                    plan.top.size() * 4 + rec_bytes;
+  if (!keep_leaves) {
+    (void)hipFree(h->leaves);
+    h->leaves = nullptr;
+  }
+  h->device_bytes = P.bytes + (keep_leaves ? leaf_bytes : 0) + rec_bytes;
   *out = h;
   return VRT_OK;
 }

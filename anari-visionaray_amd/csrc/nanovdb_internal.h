@@ -5,21 +5,22 @@
 #include <stdint.h>
 
 #include "abi_internal.h"
+#include "kernel_common.h"
 
 struct vrt_nanovdb_s {
   int device = 0;
   hipStream_t stream = nullptr;  // the creating context's stream (not used after destroy)
-  // device, for lookups: slot table, with its region table where it is not
-  // dense, records of 9^3 voxels, constants (background first); see KVolume
+  // device allocations: tables (the pointers after these three point into
+  // it), leaf values (null where the records hold all of them), records
+  char *mem = nullptr;
+  float *leaves = nullptr;
+  float *recs = nullptr;  // records of 9^3 voxels
+  // for lookups: slot table, with its region table where it is not dense
+  // (see KVolume)
   int32_t *table = nullptr;
   int32_t *region_top = nullptr;
-  float *recs = nullptr;
-  float *consts = nullptr;
   int slo[3] = {0, 0, 0}, sn[3] = {0, 0, 0};
-  // device, for value ranges: top table over 128^3 regions (block index >= 0,
-  // or -1 - constant), per-slot value ranges of the blocks (float2)
-  int32_t *top = nullptr;
-  float *slot_ranges = nullptr;
+  const vrt::KNvTree *tree = nullptr;  // the tree's tables (constants: background first)
   int lo[3] = {0, 0, 0}, n[3] = {0, 0, 0};  // top-table origin (in 128-voxel units) / dims
   uint64_t block_count = 0;
   float inv_f[9], vec_f[3];                  // Map::mInvMatF, mVecF

@@ -40,14 +40,7 @@ int pathtrace_blocks_per_cu(const KScene &sc, size_t lds_bytes, bool nrc = false
                             bool grad = false);
 hipError_t launch_bricks(const float *lin, const int dims[3], float *bricks, hipStream_t s);
 hipError_t launch_value_ranges(const KVolume &v, float *ranges, hipStream_t s);
-// The NanoVDB tree as two device tables (see nanovdb_field.cpp): top table
-// over 128^3 regions, blocks of 16^3 slots, constants, leaf values
-struct KNvTree {
-  const int32_t *top, *blocks;
-  const float *consts, *leaves;
-  int lo[3], n[3];
-};
-// The lookup table built from it: `entries` slot entries, dense over [lo, lo
+// The lookup table built from a NanoVDB tree: `entries` slot entries, dense over [lo, lo
 // + n) slots, or (region_of_block given) blocks of 16^3 over [lo, lo + n)
 // regions, block b covering region region_of_block[b] (x-fastest index)
 struct KNvTable {
@@ -56,10 +49,11 @@ struct KNvTable {
   size_t entries;
   int lo[3], n[3];
 };
-// fills the table: a constant where the slot and its 7 upper neighbours hold
-// the same one, else the next record; *records (zeroed by the caller) counts
-hipError_t launch_nanovdb_table(const KNvTree &t, const KNvTable &T, uint32_t *records,
-                                hipStream_t s);
+// fills the table: where the slot or one of its 7 upper neighbours holds a
+// leaf the next record (kNvTreeEntry without `use_records`), else their constant, or
+// kNvTreeEntry where they hold several.  *records (zeroed by the caller) counts
+hipError_t launch_nanovdb_table(const KNvTree &t, const KNvTable &T, bool use_records,
+                                uint32_t *records, hipStream_t s);
 // fills the records the table names
 hipError_t launch_nanovdb_records(const KNvTree &t, const KNvTable &T, float *recs,
                                   hipStream_t s);

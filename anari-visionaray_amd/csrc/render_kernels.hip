@@ -304,8 +304,8 @@ __device__ inline float sample_structured(const KVolume &v, f3 P) {
 // a slot comparison, look-up and branch for each of 7 taps) the cloud 320^3
 // at 1080p took 11.3 ms a frame, now 5.9 ms.
 // ---------------------------------------------------------------------------
-// entry of the 8^3 slot (sx, sy, sz) (voxel index >> 3): >= 0 record, else
-// -1 - constant index
+// entry of the 8^3 slot (sx, sy, sz) (voxel index >> 3): >= 0 record,
+// kNvTreeEntry or -1 - constant index
 __device__ inline int nvdb_entry(const KVolume &v, int sx, int sy, int sz) {
   const int shift = v.nv_rtop ? 4 : 0;
   const int tx = (sx >> shift) - v.nv_slo[0], ty = (sy >> shift) - v.nv_slo[1],
@@ -320,6 +320,22 @@ __device__ inline int nvdb_entry(const KVolume &v, int sx, int sy, int sz) {
   const int t = v.nv_rtop[s];
   if (t < 0) return t;
   return v.nv_tab[size_t(t) * 4096u + uint32_t((((sz & 15) << 4) | (sy & 15)) << 4 | (sx & 15))];
+}
+
+// entry of a slot in the tree tables (>= 0 leaf, else -1 - constant)
+__device__ inline int nvtree_slot(const KNvTree &v, int sx, int sy, int sz) {
+  const int tx = (sx >> 4) - v.lo[0], ty = (sy >> 4) - v.lo[1], tz = (sz >> 4) - v.lo[2];
+  if (uint32_t(tx) >= uint32_t(v.n[0]) || uint32_t(ty) >= uint32_t(v.n[1]) ||
+      uint32_t(tz) >= uint32_t(v.n[2]))
+    return -1;  // background
+  const int t = v.top[(size_t(tz) * size_t(v.n[1]) + size_t(ty)) * size_t(v.n[0]) + tx];
+  if (t < 0) return t;
+  return v.blocks[size_t(t) * 4096u + uint32_t((((sz & 15) << 4) | (sy & 15)) << 4 | (sx & 15))];
+}
+__device__ inline float nvtree_value(const KNvTree &v, int i, int j, int k) {
+  const int e = nvtree_slot(v, i >> 3, j >> 3, k >> 3);
+  return e >= 0 ? v.leaves[size_t(e) * 512u + uint32_t(((i & 7) << 6) | ((j & 7) << 3) | (k & 7))]
+                : v.consts[-1 - e];
 }
 
 // createSampler<1|0>(acc)(worldToIndexF(P)): the map is an fmaf chain over
@@ -345,7 +361,32 @@ __device__ inline float sample_nanovdb(const KVolume &v, f3 P) {
   const int e = nvdb_entry(v, i >> 3, j >> 3, k >> 3);
   if (e < 0) {
     float c = v.nv_bg;
-    if (e != -1) c = v.nv_consts[-1 - e];
+    if (e != -1) {
+      const KNvTree &tree = *v.nv_tree;
+      if (e == kNvTreeEntry) {
+        // one tap after the other, z fastest: few lookups come here, and the
+        // taps at once would cost the others registers
+        float z0 = 0.f, y0 = 0.f, x0 = 0.f;
+#pragma unroll 1
+        for (int n = 0;; ++n) {
+          float t = nvtree_value(tree, i + (n >> 2), j + ((n >> 1) & 1), k + (n & 1));
+          if (nearest) return t;
+          if (!(n & 1)) {
+            z0 = t;
+            continue;
+          }
+          t = lerpf(z0, t, w[2]);
+          if (!(n & 2)) {
+            y0 = t;
+            continue;
+          }
+          t = lerpf(y0, t, w[1]);
+          if (n & 4) return lerpf(x0, t, w[0]);
+          x0 = t;
+        }
+      }
+      c = tree.consts[-1 - e];
+    }
     // lerp(c, c, w): c, NaN for an infinite or NaN constant or weight
     return nearest ? c : c + (w[0] + w[1] + w[2]) * (c - c);
   }
@@ -493,8 +534,10 @@ __device__ inline bool sample_field(const KVolume &v, f3 P, float &value) {
 // P +- delta along each axis, false unless all six samples have a value.
 // The gradient normal is its normalisation; a zero gradient (a flat region)
 // gives no normal here -- the reference's normalize(0) is NaN.
+// (Inlined by force: left as a call in the largest variants, its volume
+// argument takes a private copy of the scene, 3 KB of scratch per lane.)
 template <int FIELD = kAnyField>
-__device__ inline f3 gradient_normal(const KVolume &v, f3 P) {
+__device__ __forceinline__ f3 gradient_normal(const KVolume &v, f3 P) {
   const f3 delta = v.S * v.cell_size;  // cellSize * diag(voxelSpaceTransform)
   float x0, x1, y0, y1, z0, z1;
   const bool b0 = sample_field<FIELD>(v, P + mk(delta.x, 0.f, 0.f), x1);
@@ -1603,7 +1646,7 @@ __device__ inline float4 light_backdrop(const KScene &sc, const KRay &ray, float
 // the ambient term.  Lights are sampled at P itself, in voxel space, as the
 // reference does.
 template <int FIELD>
-__device__ inline f3 gradient_shade(const KScene &sc, const KVolume &v, const KParams &P, f3 Pv,
+__device__ __forceinline__ f3 gradient_shade(const KScene &sc, const KVolume &v, const KParams &P, f3 Pv,
                                     f3 viewDir, f3 albedo, uint32_t &rs) {
   f3 gn = gradient_normal<FIELD>(v, Pv);
   gn = faceforward(gn, viewDir, gn);
@@ -3056,23 +3099,6 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// nanovdb tree tables: entry of a slot (>= 0 leaf, else -1 - constant), value
-// of a voxel
-__device__ inline int nvtree_slot(const KNvTree &v, int sx, int sy, int sz) {
-  const int tx = (sx >> 4) - v.lo[0], ty = (sy >> 4) - v.lo[1], tz = (sz >> 4) - v.lo[2];
-  if (uint32_t(tx) >= uint32_t(v.n[0]) || uint32_t(ty) >= uint32_t(v.n[1]) ||
-      uint32_t(tz) >= uint32_t(v.n[2]))
-    return -1;  // background
-  const int t = v.top[(size_t(tz) * size_t(v.n[1]) + size_t(ty)) * size_t(v.n[0]) + tx];
-  if (t < 0) return t;
-  return v.blocks[size_t(t) * 4096u + uint32_t((((sz & 15) << 4) | (sy & 15)) << 4 | (sx & 15))];
-}
-__device__ inline float nvtree_value(const KNvTree &v, int i, int j, int k) {
-  const int e = nvtree_slot(v, i >> 3, j >> 3, k >> 3);
-  return e >= 0 ? v.leaves[size_t(e) * 512u + uint32_t(((i & 7) << 6) | ((j & 7) << 3) | (k & 7))]
-                : v.consts[-1 - e];
-}
-
 // slot coordinates of table entry i
 __device__ inline void nvtable_slot(const KNvTable &T, size_t i, int &x, int &y, int &z) {
   const size_t r = T.region_of_block ? size_t(T.region_of_block[i >> 12]) : i;
@@ -3086,42 +3112,53 @@ __device__ inline void nvtable_slot(const KNvTable &T, size_t i, int &x, int &y,
   }
 }
 
-// One thread per table entry: a slot whose 9^3 voxels (its own 8^3 and the
-// first layers of its 7 upper neighbours) lie in one constant keeps that,
-// every other slot gets a record.
+// One thread per table entry (see nanovdb_field.cpp for the kinds of entry);
+// the grid strides, as tables may have more entries than a grid has threads.
+constexpr size_t kNvTableBlocks = size_t(1) << 20;
+
 __global__ void __launch_bounds__(256)
-    k_nvdb_table(KNvTree t, KNvTable T, uint32_t *__restrict__ records) {
-  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const bool in = i < T.entries;
-  int e = -1;
-  bool need = false;
-  if (in) {
-    int x, y, z;
-    nvtable_slot(T, i, x, y, z);
-    e = nvtree_slot(t, x, y, z);
-    need = e >= 0;
-    for (int k = 1; k < 8 && !need; ++k)
-      need = nvtree_slot(t, x + (k & 1), y + ((k >> 1) & 1), z + (k >> 2)) != e;
+    k_nvdb_table(KNvTree t, KNvTable T, bool use_records, uint32_t *__restrict__ records) {
+  for (size_t base = size_t(blockIdx.x) * 256; base < T.entries; base += size_t(gridDim.x) * 256) {
+    const size_t i = base + threadIdx.x;
+    const bool in = i < T.entries;
+    int e = -1;
+    bool leaf = false, differ = false;
+    if (in) {
+      int x, y, z;
+      nvtable_slot(T, i, x, y, z);
+      e = nvtree_slot(t, x, y, z);
+      leaf = e >= 0;
+      for (int k = 1; k < 8 && !leaf; ++k) {
+        const int o = nvtree_slot(t, x + (k & 1), y + ((k >> 1) & 1), z + (k >> 2));
+        leaf = o >= 0;
+        differ = differ || o != e;
+      }
+    }
+    const uint32_t r = wave_claim(records, leaf && use_records);
+    if (in) T.table[i] = leaf ? (use_records ? int(r) : kNvTreeEntry) : differ ? kNvTreeEntry : e;
   }
-  const uint32_t r = wave_claim(records, need);
-  if (in) T.table[i] = need ? int(r) : e;
 }
 
-// One wave per 64 table entries: fills their records (x fastest, rows of 9,
-// zero padding)
+// One wave per `share` (at most 64) table entries: fills their records (x
+// fastest, rows of 9, zero padding).  A wave fills one record after the other,
+// each a few round trips, so small tables give a wave few entries: the grid of
+// a 64^3 cloud is created in 0.31 ms (64 entries a wave: 0.63 ms).
 __global__ void __launch_bounds__(256)
-    k_nvdb_records(KNvTree t, KNvTable T, float *__restrict__ recs) {
+    k_nvdb_records(KNvTree t, KNvTable T, int share, float *__restrict__ recs) {
   const int lane = int(threadIdx.x) & 63;
-  const size_t base = (size_t(blockIdx.x) * 4 + (threadIdx.x >> 6)) * 64;
-  const int mine = base + lane < T.entries ? T.table[base + lane] : -1;
-  for (unsigned long long m = __ballot(mine >= 0); m; m &= m - 1) {
-    const int src = __ffsll(m) - 1;
-    const int e = __shfl(mine, src, 64);
-    int x, y, z;
-    nvtable_slot(T, base + src, x, y, z);
-    float *dst = recs + size_t(e) * VRT_BRICK_FLOATS;
-    for (int l = lane; l < VRT_BRICK_FLOATS; l += 64)
-      dst[l] = l < 729 ? nvtree_value(t, 8 * x + l % 9, 8 * y + (l / 9) % 9, 8 * z + l / 81) : 0.f;
+  for (size_t base = (size_t(blockIdx.x) * 4 + (threadIdx.x >> 6)) * share; base < T.entries;
+       base += size_t(gridDim.x) * 4 * share) {
+    const int mine = lane < share && base + lane < T.entries ? T.table[base + lane] : -1;
+    for (unsigned long long m = __ballot(mine >= 0); m; m &= m - 1) {
+      const int src = __ffsll(m) - 1;
+      const int e = __shfl(mine, src, 64);
+      int x, y, z;
+      nvtable_slot(T, base + src, x, y, z);
+      float *dst = recs + size_t(e) * VRT_BRICK_FLOATS;
+      for (int l = lane; l < VRT_BRICK_FLOATS; l += 64)
+        dst[l] =
+            l < 729 ? nvtree_value(t, 8 * x + l % 9, 8 * y + (l / 9) % 9, 8 * z + l / 81) : 0.f;
+    }
   }
 }
 
@@ -3157,23 +3194,22 @@ __global__ void __launch_bounds__(256)
   const int c = int(blockIdx.x * blockDim.x + threadIdx.x);
   if (c >= ncells) return;
   const int32_t *b = cell_voxels + 6 * size_t(c);
-  const float2 *slot_ranges = reinterpret_cast<const float2 *>(v.nv_slot_ranges);
+  const KNvTree T = *v.nv_tree;
   float mn = FLT_MAX, mx = -FLT_MAX;
   for (int sz = b[2] >> 3; sz <= (b[5] >> 3); ++sz)
     for (int sy = b[1] >> 3; sy <= (b[4] >> 3); ++sy)
       for (int sx = b[0] >> 3; sx <= (b[3] >> 3); ++sx) {
-        const int tx = (sx >> 4) - v.nv_lo[0], ty = (sy >> 4) - v.nv_lo[1],
-                  tz = (sz >> 4) - v.nv_lo[2];
+        const int tx = (sx >> 4) - T.lo[0], ty = (sy >> 4) - T.lo[1], tz = (sz >> 4) - T.lo[2];
         float lo, hi;
         int t = -1;
-        if (uint32_t(tx) < uint32_t(v.nv_n[0]) && uint32_t(ty) < uint32_t(v.nv_n[1]) &&
-            uint32_t(tz) < uint32_t(v.nv_n[2]))
-          t = v.nv_top[(size_t(tz) * v.nv_n[1] + ty) * v.nv_n[0] + tx];
+        if (uint32_t(tx) < uint32_t(T.n[0]) && uint32_t(ty) < uint32_t(T.n[1]) &&
+            uint32_t(tz) < uint32_t(T.n[2]))
+          t = T.top[(size_t(tz) * T.n[1] + ty) * T.n[0] + tx];
         if (t < 0) {
-          lo = hi = v.nv_consts[-1 - t];
+          lo = hi = T.consts[-1 - t];
         } else {
-          const float2 r =
-              slot_ranges[size_t(t) * 4096u + uint32_t((((sz & 15) << 4) | (sy & 15)) << 4 | (sx & 15))];
+          const float2 r = T.slot_ranges[size_t(t) * 4096u +
+                                         uint32_t((((sz & 15) << 4) | (sy & 15)) << 4 | (sx & 15))];
           lo = r.x;
           hi = r.y;
         }
@@ -3622,19 +3658,22 @@ hipError_t launch_tet_planes(const uint32_t *start, const float4 *recs, const fl
   return hipGetLastError();
 }
 
-hipError_t launch_nanovdb_table(const KNvTree &t, const KNvTable &T, uint32_t *records,
-                                hipStream_t s) {
+hipError_t launch_nanovdb_table(const KNvTree &t, const KNvTable &T, bool use_records,
+                                uint32_t *records, hipStream_t s) {
   if (T.entries == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_nvdb_table, dim3(unsigned((T.entries + 255) / 256)), dim3(256), 0, s, t, T,
-                     records);
+  hipLaunchKernelGGL(k_nvdb_table, dim3(unsigned(std::min((T.entries + 255) / 256, kNvTableBlocks))),
+                     dim3(256), 0, s, t, T, use_records, records);
   return hipGetLastError();
 }
 
 hipError_t launch_nanovdb_records(const KNvTree &t, const KNvTable &T, float *recs,
                                   hipStream_t s) {
   if (T.entries == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_nvdb_records, dim3(unsigned((T.entries + 255) / 256)), dim3(256), 0, s, t,
-                     T, recs);
+  // 16,384 waves, twice what the chip holds, before a wave takes more entries
+  const int share = int(std::min<size_t>(std::max<size_t>(T.entries / 16384, 1), 64));
+  const size_t blocks = (T.entries + 4 * share - 1) / (4 * share);
+  hipLaunchKernelGGL(k_nvdb_records, dim3(unsigned(std::min(blocks, kNvTableBlocks))), dim3(256), 0,
+                     s, t, T, share, recs);
   return hipGetLastError();
 }
 

@@ -106,14 +106,10 @@ int make_nanovdb_volume(const vrt_volume &in, int lds_offset, KVolume &v) {
   v.nv_tab = g->table;
   v.nv_rtop = g->region_top;
   v.nv_bg = g->background;
-  v.nv_top = g->top;
-  v.nv_consts = g->consts;
-  v.nv_slot_ranges = g->slot_ranges;
+  v.nv_tree = g->tree;
   for (int a = 0; a < 3; ++a) {
     v.nv_slo[a] = g->slo[a];
     v.nv_sn[a] = g->sn[a];
-    v.nv_lo[a] = g->lo[a];
-    v.nv_n[a] = g->n[a];
     v.nv_vec[a] = g->vec_f[a];
   }
   for (int i = 0; i < 9; ++i) v.nv_inv[i] = g->inv_f[i];

@@ -359,7 +359,7 @@ typedef struct vrt_nanovdb_info {
   uint64_t leaves;                  /* leaves inside the bounds */
   uint64_t constants;               /* distinct constants (background first) */
   uint64_t active_voxels;           /* TreeData::mVoxelCount */
-  uint64_t device_bytes;            /* tables + records + constants + slot ranges */
+  uint64_t device_bytes;            /* tables, and records or leaf values */
 } vrt_nanovdb_info;
 
 VRT_API int vrt_nanovdb_create(vrt_context ctx, const void *grid_buffer, uint64_t bytes,
