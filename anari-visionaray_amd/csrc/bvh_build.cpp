@@ -62,8 +62,40 @@ struct Builder {
   std::vector<int> order;
   std::vector<Node2> nodes;
   uint32_t depth = 0;
+  int longest = 0;  // leaf
+  // the sweep ends at level `deepest` (it may peel off a few items per level);
+  // lists longer than kMaxLeaf left there are kept as leaves, halved, or chained
+  enum Lists { kKeep, kHalve, kChain } lists = kKeep;
+  uint32_t deepest = 60;
+  static constexpr int kMaxLeaf = 255;
 
   Builder(const std::vector<Box> &b, const std::vector<float> &c) : tri_box(b), centre(c) {}
+
+  // Makes node `id` the head of a chain: one leaf after the other beside the
+  // rest of the list.  No node of it has two inner children, so a traversal
+  // stacks nothing on the way down (halves stack up to 3 nodes per 4-wide
+  // level).
+  void build_chain(int id, int first, int count) {
+    const int links = (count + kMaxLeaf - 1) / kMaxLeaf;
+    depth += uint32_t(links);
+    std::vector<Box> own(static_cast<size_t>(links));
+    for (int i = 0; i < count; ++i) own[size_t(i / kMaxLeaf)].grow(tri_box[order[first + i]]);
+    std::vector<Box> rest(own);
+    for (int k = links - 2; k >= 0; --k) rest[size_t(k)].grow(rest[size_t(k) + 1]);
+    for (int k = 0; k < links - 1; ++k) {
+      const int leaf = int(nodes.size());
+      nodes.resize(nodes.size() + 2);
+      nodes[leaf].box = own[size_t(k)];
+      nodes[leaf].first = first + k * kMaxLeaf;
+      nodes[leaf].count = kMaxLeaf;
+      nodes[leaf + 1].box = rest[size_t(k) + 1];
+      nodes[id].left = leaf;
+      nodes[id].right = leaf + 1;
+      id = leaf + 1;
+    }
+    nodes[id].first = first + (links - 1) * kMaxLeaf;
+    nodes[id].count = count - (links - 1) * kMaxLeaf;
+  }
 
   int build(int first, int count, uint32_t level) {
     depth = std::max(depth, level + 1);
@@ -78,18 +110,21 @@ struct Builder {
     auto make_leaf = [&]() {
       nodes[id].first = first;
       nodes[id].count = count;
+      longest = std::max(longest, count);
       return id;
     };
-    // below level 60 (a sweep that peels off a few triangles per level) lists
-    // are halved; the traversal holds a leaf's count in a byte
-    const bool halve = level >= 60;
-    if (count <= 4 || (halve && count <= 255)) return make_leaf();
+    const bool deep = level >= deepest;
+    if (count <= 4 || (deep && (lists == kKeep || count <= kMaxLeaf))) return make_leaf();
+    if (deep && lists == kChain) {
+      build_chain(id, first, count);
+      return id;
+    }
     int axis = 0;
     for (int a = 1; a < 3; ++a)
       if (cbox.hi[a] - cbox.lo[a] > cbox.hi[axis] - cbox.lo[axis]) axis = a;
     const float ext = cbox.hi[axis] - cbox.lo[axis];
     int mid = -1;
-    if (ext > 0.f && !halve) {
+    if (ext > 0.f && !deep) {
       constexpr int kBins = 16;
       Box bb[kBins];
       int bn[kBins] = {0};
@@ -230,6 +265,37 @@ uint32_t stack_need(const std::vector<float4> &nodes4) {
   return nn ? need[0] : 0u;
 }
 
+// Builds the tree over all items and collapses it; returns the most entries a
+// traversal can stack (more than it holds: refused).  `short_leaves`: the
+// traversal holds a leaf's count in a byte.  Whether a tree is accepted is
+// decided with long lists as leaves; these are then halved where that fits the
+// stack, else chained, from a level at which it fits (a chain from level 0
+// stacks nothing).
+uint32_t build_nodes(Builder &B, bool short_leaves, std::vector<float4> &nodes4,
+                     std::vector<int> &leaf_items) {
+  const size_t n = B.tri_box.size();
+  auto build = [&](Builder::Lists lists, uint32_t deepest) {
+    B.lists = lists;
+    B.deepest = deepest;
+    B.longest = 0;
+    B.depth = 0;
+    B.nodes.clear();
+    nodes4.clear();
+    leaf_items.clear();
+    B.order.resize(n);
+    for (size_t i = 0; i < n; ++i) B.order[i] = int(i);
+    B.build(0, int(n), 0);
+    collapse4(B, nodes4, leaf_items);
+    return stack_need(nodes4);
+  };
+  uint32_t need = build(Builder::kKeep, 60);
+  if (!short_leaves || B.longest <= Builder::kMaxLeaf || need > VRT_BVH_MAX_STACK) return need;
+  need = build(Builder::kHalve, 60);
+  for (uint32_t level = 60; need > VRT_BVH_MAX_STACK; level -= 12)
+    need = build(Builder::kChain, level);
+  return need;
+}
+
 }  // namespace
 
 extern "C" {
@@ -267,14 +333,10 @@ int vrt_bvh_build(vrt_context ctx, const float *vertices, int64_t num_vertices,
     for (int a = 0; a < 3; ++a) centre[3 * i + a] = 0.5f * (boxes[i].lo[a] + boxes[i].hi[a]);
   }
   Builder B(boxes, centre);
-  B.order.resize(n);
-  for (size_t i = 0; i < n; ++i) B.order[i] = int(i);
   B.nodes.reserve(2 * n / 4 + 16);
-  B.build(0, int(n), 0);
-
   std::vector<float4> nodes4;
   std::vector<int> leaf_items;
-  collapse4(B, nodes4, leaf_items);
+  const uint32_t stack_bound = build_nodes(B, true, nodes4, leaf_items);
   std::vector<float4> tris_out;
   tris_out.reserve(3 * n);
   for (const int t : leaf_items) {
@@ -286,7 +348,6 @@ int vrt_bvh_build(vrt_context ctx, const float *vertices, int64_t num_vertices,
     tris_out.push_back(make_float4(p[3], p[4], p[5], 0.f));
     tris_out.push_back(make_float4(p[6], p[7], p[8], 0.f));
   }
-  const uint32_t stack_bound = stack_need(nodes4);
   if (stack_bound > VRT_BVH_MAX_STACK)
     return fail(VRT_ERROR_UNSUPPORTED,
                 "bvh: a traversal of this tree can stack %u entries, the kernels hold %d "
@@ -417,13 +478,9 @@ int vrt_tls_build(vrt_context ctx, const vrt_instance *ins, int n, vrt_tls *out)
     }
   }
   Builder B(boxes, centre);
-  B.order.resize(size_t(n));
-  for (int i = 0; i < n; ++i) B.order[size_t(i)] = i;
-  B.build(0, n, 0);
   std::vector<float4> nodes4;
   std::vector<int> leaf_items;
-  collapse4(B, nodes4, leaf_items);
-  const uint32_t stack_bound = stack_need(nodes4);
+  const uint32_t stack_bound = build_nodes(B, false, nodes4, leaf_items);
   if (stack_bound > VRT_BVH_MAX_STACK)
     return fail(VRT_ERROR_UNSUPPORTED, "tls: a walk of this tree can stack %u entries, the "
                 "kernels hold %d", stack_bound, VRT_BVH_MAX_STACK);

@@ -77,3 +77,60 @@ def test_any_hit_returns_the_first_of_a_leaf(pkg, gpu_ctx, count):
     got = keep & (first >= 0)
     np.testing.assert_allclose(t[got], np.abs(r[got, 2] + first[got]), rtol=1e-5)
     assert got.sum() > 300
+
+
+def test_long_lists_where_halves_exceed_the_stack(pkg, oracle, gpu_ctx):
+    """Clusters at 2^-i fill the traversal's stack on the way to level 60,
+    below which 60,000 triangles are left: the tree with that list as one leaf
+    stacks 52 entries, its halves 69 of the 64 that traversals hold."""
+    vrt = pkg.vrt
+    rng = np.random.default_rng(0)
+    s = np.concatenate([np.repeat(2.0 ** -np.arange(110), 14), np.full(60000, 2.0 ** -110)])
+    c = s[:, None] * (np.array([1.0, 0, 0]) + 0.2 * rng.random((len(s), 3)))
+    tri = (c[:, None] + s[:, None, None] * 0.01 * rng.random((len(s), 3, 3))).astype(np.float32)
+    v = tri.reshape(-1, 3)
+    mesh = vrt.DeviceMesh(gpu_ctx, v, None, "sah")
+    assert mesh.info.stack_bound <= 64 and mesh.info.depth > 69
+    scene = vrt.make_scene([], [], [(mesh, (0.7, 0.7, 0.7))])
+    r = np.zeros((3000, 8), np.float32)
+    k = rng.integers(0, 14 * 40, 3000)  # at triangles of the first 40 scales
+    d = rng.normal(size=(3000, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    r[:, 3:6] = d
+    r[:, :3] = tri[k].mean(1) - 3 * s[k, None] * d
+    r[:, 7] = 1e30
+    om = oracle.OracleMesh(v, None)
+    t, p = vrt.intersect_surfaces(gpu_ctx, scene, r, False)
+    to, po = oracle.mesh_intersect(om, r, any_hit=False, brute=True)
+    np.testing.assert_array_equal(p, po)
+    np.testing.assert_array_equal(t, to)
+    assert (po >= 0).mean() > 0.5
+    _, pa = vrt.intersect_surfaces(gpu_ctx, scene, r, True)
+    np.testing.assert_array_equal(pa >= 0, po >= 0)
+
+
+def test_long_lists_of_instances(pkg, gpu_ctx):
+    """Instance trees hold lists of any length below level 60 as leaves, as the
+    instance walk reads whole counts."""
+    vrt = pkg.vrt
+    rng = np.random.default_rng(1)
+    tri = np.array([(-0.5, -0.5, 0), (0.5, -0.5, 0), (0, 0.5, 0)], np.float32)
+    mesh = vrt.DeviceMesh(gpu_ctx, tri, None, "sah")
+    s = np.concatenate([2.0 ** -np.arange(90), np.full(400, 2.0 ** -90)])
+    xf = np.zeros((len(s), 3, 4), np.float32)
+    xf[:, [0, 1, 2], [0, 1, 2]] = 0.05
+    xf[:, 0, 3] = s * (1 + 0.2 * rng.random(len(s)))
+    tls = vrt.DeviceTls(gpu_ctx, [(mesh, x, (0.7, 0.7, 0.7)) for x in xf])
+    assert tls.info.stack_bound <= 8
+    scene = vrt.make_scene([], [], [], tls=tls)
+    r = np.zeros((600, 8), np.float32)
+    r[:, 0] = rng.uniform(-0.1, 1.3, 600)
+    r[:, 1] = rng.uniform(-0.03, 0.03, 600)
+    r[:, 2], r[:, 5], r[:, 7] = 1.0, -1.0, 1e30
+    _, p = vrt.intersect_surfaces(gpu_ctx, scene, r, True)
+    x = (r[:, None, 0] - xf[None, :, 0, 3]) / 0.05
+    y = r[:, None, 1] / 0.05
+    margin = np.minimum(y + 0.5, 0.5 - y - 2 * np.abs(x)).max(1)  # > 0: inside one
+    clear = np.abs(margin) > 1e-3
+    np.testing.assert_array_equal(p[clear] >= 0, margin[clear] > 0)
+    assert 50 < (margin > 0).sum() < 550
