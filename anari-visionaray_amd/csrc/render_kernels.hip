@@ -2887,18 +2887,27 @@ __global__ void __launch_bounds__(256)
 }
 
 // Value range of each macrocell: min/max over every voxel a trilinear sample
-// inside the cell can read (see vrt_build_value_ranges).  One workgroup per
-// macrocell; each wave reads as many voxel rows of the footprint side by side
-// as fit in its 64 lanes (18-voxel rows of a 16^3 cell: 3), so a lane keeps
-// its x and steps y and z by additions.  384x320x250 voxels, 16^3 cells:
-// 51 us; one linear index split by two divisions per voxel took 114 us.
+// inside the cell can read (see vrt_build_value_ranges).  WAVES waves share a
+// cell: a workgroup's four, or one where there are many small cells (see
+// launch_value_ranges).
+// Each wave reads as many voxel rows of the footprint side by side as fit in
+// its 64 lanes (18-voxel rows of a 16^3 cell: 3), so a lane keeps its x and
+// steps y and z by additions, with several rows in flight.
+// Bound by memory for large cells (384x320x250 voxels, 16^3 cells: 46 us; one
+// linear index split by two divisions per voxel: 99), by the set-up of each
+// cell for small ones (512^3 voxels, 4^3 cells: 1.47 ms; four waves with 9
+// rows in flight 6.30, the linear index 3.62).
+template <int WAVES>
 __global__ void __launch_bounds__(256)
-    k_value_ranges(KVolume v, float2 *__restrict__ ranges) {
+    k_value_ranges(KVolume v, int cells, float2 *__restrict__ ranges) {
   const int G0 = v.gdims[0], G1 = v.gdims[1], G2 = v.gdims[2];
-  const int mc = blockIdx.x;
-  const int m[3] = {mc % G0, (mc / G0) % G1, mc / (G0 * G1)};
-  const int G[3] = {G0, G1, G2};
+  const int lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6;
+  const int mc = WAVES == 1 ? int(blockIdx.x) * 4 + wave : int(blockIdx.x);
+  if (WAVES == 1 && mc >= cells) return;
+  const int mx = mc % G0, my = (mc / G0) % G1, mz = mc / (G0 * G1);
   int lo[3], hi[3];
+  const int m[3] = {mx, my, mz};
+  const int G[3] = {G0, G1, G2};
   for (int a = 0; a < 3; ++a) {
     const double c0 = double(m[a]) * v.dims[a] / G[a] - 0.5;
     const double c1 = double(m[a] + 1) * v.dims[a] / G[a] - 0.5;
@@ -2906,17 +2915,16 @@ __global__ void __launch_bounds__(256)
     hi[a] = min(v.dims[a] - 1, int(floor(c1)) + 1);
   }
   const int ex = hi[0] - lo[0] + 1, ey = hi[1] - lo[1] + 1, ez = hi[2] - lo[2] + 1;
-  const int lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6;
   const int cols = min(ex, 64), per_wave = 64 / cols;  // rows side by side in a wave
   const int sub = lane / cols;
-  const int step = 4 * per_wave, dz = step / ey, dy = step - dz * ey;
-  const int r0 = wave * per_wave + sub;
+  const int step = WAVES * per_wave, dz = step / ey, dy = step - dz * ey;
+  const int r0 = (WAVES == 1 ? 0 : wave * per_wave) + sub;
   float vmin = FLT_MAX, vmax = -FLT_MAX;
   for (int x = lane - sub * cols; sub < per_wave && x < ex; x += cols) {
     const int xi = lo[0] + x;
     const float *bx = v.bricks + size_t(xi >> 3) * VRT_BRICK_FLOATS + size_t(xi & 7);
     int y = r0 % ey, z = r0 / ey;
-    constexpr int kRows = 9;  // rows in flight per lane
+    constexpr int kRows = WAVES == 1 ? 4 : 9;  // rows in flight per lane
     while (z < ez) {
       float val[kRows];
 #pragma unroll
@@ -2944,15 +2952,19 @@ __global__ void __launch_bounds__(256)
     vmin = fminf(vmin, __shfl_xor(vmin, o, 64));
     vmax = fmaxf(vmax, __shfl_xor(vmax, o, 64));
   }
-  __shared__ float smin[4], smax[4];
-  if (lane == 0) {
-    smin[wave] = vmin;
-    smax[wave] = vmax;
+  if constexpr (WAVES == 1) {
+    if (lane == 0) ranges[mc] = make_float2(vmin, vmax);
+  } else {
+    __shared__ float smin[4], smax[4];
+    if (lane == 0) {
+      smin[wave] = vmin;
+      smax[wave] = vmax;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+      ranges[mc] = make_float2(fminf(fminf(smin[0], smin[1]), fminf(smin[2], smin[3])),
+                               fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3])));
   }
-  __syncthreads();
-  if (threadIdx.x == 0)
-    ranges[mc] = make_float2(fminf(fminf(smin[0], smin[1]), fminf(smin[2], smin[3])),
-                             fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3])));
 }
 
 // Atomic min / max of floats through their order-preserving integer images:
@@ -3641,8 +3653,18 @@ hipError_t launch_bricks(const float *lin, const int dims[3], float *bricks, hip
 
 hipError_t launch_value_ranges(const KVolume &v, float *ranges, hipStream_t s) {
   const int nmc = v.gdims[0] * v.gdims[1] * v.gdims[2];
-  hipLaunchKernelGGL(k_value_ranges, dim3(nmc), dim3(256), 0, s, v,
-                     reinterpret_cast<float2 *>(ranges));
+  // One wave per cell where these fill the chip (8,192 waves) and a footprint
+  // (16^3 voxels: 14^3 cells) is no long walk for it, and for the smallest:
+  // with one / four waves 13,824 cells of 10^3 voxels take 28 / 45 us, 8,000 of
+  // 14^3 35 / 38, 7,680 of 16^3 49 / 46, 512 of 8^3 4.8 / 4.2
+  double footprint = 1;
+  for (int a = 0; a < 3; ++a) footprint *= double(v.dims[a]) / v.gdims[a] + 2;
+  const bool one = footprint <= (nmc >= 4096 ? 4096 : 256);
+  float2 *out = reinterpret_cast<float2 *>(ranges);
+  if (one)
+    hipLaunchKernelGGL(k_value_ranges<1>, dim3((nmc + 3) / 4), dim3(256), 0, s, v, nmc, out);
+  else
+    hipLaunchKernelGGL(k_value_ranges<4>, dim3(nmc), dim3(256), 0, s, v, nmc, out);
   return hipGetLastError();
 }
 

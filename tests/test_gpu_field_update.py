@@ -60,3 +60,24 @@ def test_bricks_ranges_majorants(pkg, gpu_ctx, dims, grid, tf_size):
             while q < 255 and f32(q) * step < m:
                 q += 1
         assert maj[c] == f32(q) * step, c
+
+
+@pytest.mark.parametrize("cell,grid", [(c, (3, 2, 2)) for c in (1, 2, 3, 4, 5, 7, 8, 11, 16, 21,
+                                                                33, 66)]
+                         + [(c, (17, 16, 16)) for c in (1, 4, 8, 14, 15)] + [(8, (17, 16, 15))])
+def test_value_ranges_of_cell_sizes(pkg, gpu_ctx, cell, grid):
+    """Footprints from 2 to 68 voxels a side, few cells and more than 4096:
+    one wave or four per cell, lanes with one row, some, and several batches."""
+    vrt = pkg.vrt
+    dims = tuple(max(1, g * cell - a) for a, g in enumerate(grid))
+    vox = np.random.default_rng(cell).normal(size=dims[::-1]).astype(np.float32)
+    dv = vrt.DeviceVolume(gpu_ctx, vox, (0, 0, 0), (1, 1, 1), np.ones((2, 4), np.float32), (0, 1),
+                          1.0, grid)
+    got = dv.ranges.download(np.float32, grid[::-1] + (2,))
+    lo = hi = vox
+    for axis in range(3):
+        f = footprints(dims[2 - axis], grid[2 - axis])
+        lo = np.stack([lo.take(range(a, e + 1), axis).min(axis) for a, e in f], axis)
+        hi = np.stack([hi.take(range(a, e + 1), axis).max(axis) for a, e in f], axis)
+    np.testing.assert_array_equal(got[..., 0], lo)
+    np.testing.assert_array_equal(got[..., 1], hi)
