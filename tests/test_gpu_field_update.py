@@ -81,3 +81,15 @@ def test_value_ranges_of_cell_sizes(pkg, gpu_ctx, cell, grid):
         hi = np.stack([hi.take(range(a, e + 1), axis).max(axis) for a, e in f], axis)
     np.testing.assert_array_equal(got[..., 0], lo)
     np.testing.assert_array_equal(got[..., 1], hi)
+
+
+@pytest.mark.parametrize("dims", [(1, 1, 1), (8, 9, 7), (16, 17, 300), (9, 1000, 200), (17, 520, 440),
+                                  (25, 400, 330), (112, 110, 112), (120, 128, 129), (100, 3, 4096)])
+def test_brick_records_of_sizes(pkg, gpu_ctx, dims):
+    """Brick records one per workgroup and in runs: either side of 3,072
+    bricks, and one to four bricks along x."""
+    vox = np.random.default_rng(dims[0]).random(dims[::-1], np.float32)
+    dv = pkg.vrt.DeviceVolume(gpu_ctx, vox, (0, 0, 0), (1, 1, 1), np.ones((2, 4), np.float32),
+                              (0, 1), 1.0)
+    exp = records(vox)
+    np.testing.assert_array_equal(dv.bricks.download(np.float32, exp.shape), exp)
