@@ -136,6 +136,7 @@ def lib():
         L.orc_nvdb_get.argtypes = [vp, ip, vp, vp]
         L.orc_nvdb_sample.argtypes = [vp, ip, vp, ip, vp]
         L.orc_nvdb_world_bbox.argtypes = [vp, vp]
+        L.orc_tet_walk.argtypes = [vp, vp, vp, C.c_int64, ip, vp, vp]
         _lib = L
     return _lib
 
@@ -173,6 +174,19 @@ def nvdb_sample(buf, xyz, order=1):
     assert lib().orc_nvdb_sample(buf.ctypes.data, len(xyz), xyz.ctypes.data, order,
                                  out.ctypes.data) == 0
     return out
+
+
+def tet_walk(positions, vertex_data, index, points):
+    """The field at `points` (NaN outside) by a walk of the product's own lists
+    without its face planes, and the longest list."""
+    pos, val = (np.ascontiguousarray(a, np.float32) for a in (positions, vertex_data))
+    idx = np.ascontiguousarray(index, np.uint32).reshape(-1, 4)
+    pts = np.ascontiguousarray(points, np.float32)
+    out = np.empty(len(pts), np.float32)
+    longest = lib().orc_tet_walk(pos.ctypes.data, val.ctypes.data, idx.ctypes.data, len(idx),
+                                 len(pts), pts.ctypes.data, out.ctypes.data)
+    assert longest > 0
+    return out, longest
 
 
 def nvdb_world_bbox(buf):
