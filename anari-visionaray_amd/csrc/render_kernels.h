@@ -66,8 +66,8 @@ hipError_t launch_nanovdb_value_ranges(const KVolume &v, const int32_t *cell_vox
                                        float *ranges, hipStream_t s);
 // unstructured: face planes of the list entries for the search's first test
 hipError_t launch_tet_planes(const uint32_t *start, const float4 *recs, const float lo[3],
-                             const float inv_cell[3], const int dims[3], uint4 *planes,
-                             hipStream_t s);
+                             const float inv_cell[3], const int dims[3], size_t entries,
+                             uint4 *planes, hipStream_t s);
 // unstructured: cell value ranges rasterized from the tetrahedra's bounding
 // boxes and value ranges (cells without one keep the empty range)
 hipError_t launch_tet_value_ranges(const KVolume &v, float *ranges, hipStream_t s);

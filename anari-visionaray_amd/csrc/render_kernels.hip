@@ -3074,21 +3074,34 @@ __global__ void __launch_bounds__(256) k_tet_value_ranges(KVolume v, float2 *__r
 // the halfs' rounding (2^-11 of |n|_1 / 2 + |d|, 2^-24 each where subnormal)
 // and three fused multiply-adds.  Extents at which L^3 leaves the normal
 // floats, or weights the halfs' range, never reject either.
-// One thread per grid cell.
+// One thread per list entry, which finds its cell in the list starts: graded
+// meshes have cells with most of the field's entries.  (A thread per cell:
+// creating a field of 384,000 tetrahedra graded towards a corner, lists up to
+// 82,944 long, took 512 ms, 126 of them here; now 386.)
 __global__ void __launch_bounds__(256)
     k_tet_planes(const uint32_t *__restrict__ start, const float4 *__restrict__ recs, f3 lo,
                  f3 inv_cell, int nx, int ny, int nz, uint4 *__restrict__ planes) {
-  const size_t c = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (c >= size_t(nx) * ny * nz) return;
-  const double width[3] = {1.0 / inv_cell.x, 1.0 / inv_cell.y, 1.0 / inv_cell.z};
-  const double centre[3] = {lo.x + (double(c % nx) + 0.5) * width[0],
-                            lo.y + (double((c / nx) % ny) + 0.5) * width[1],
-                            lo.z + (double(c / (size_t(nx) * ny)) + 0.5) * width[2]};
-  const double cell_diag =
-      sqrt(width[0] * width[0] + width[1] * width[1] + width[2] * width[2]);
-  const double u = 5.9604644775390625e-8;  // 2^-24
-  const double q_error = 4.0 * u * fmax(double(nx), fmax(double(ny), double(nz)));
-  for (uint32_t i = start[c]; i < start[c + 1]; ++i) {
+  const size_t cells = size_t(nx) * ny * nz, entries = start[cells];
+  for (size_t i = size_t(blockIdx.x) * 256 + threadIdx.x; i < entries;
+       i += size_t(gridDim.x) * 256) {
+    size_t c = 0;  // the last cell whose list starts at or before i
+    for (size_t n = cells; n > 1;) {
+      const size_t half = n / 2;
+      if (start[c + half] <= i) {
+        c += half;
+        n -= half;
+      } else {
+        n = half;
+      }
+    }
+    const double width[3] = {1.0 / inv_cell.x, 1.0 / inv_cell.y, 1.0 / inv_cell.z};
+    const double centre[3] = {lo.x + (double(c % nx) + 0.5) * width[0],
+                              lo.y + (double((c / nx) % ny) + 0.5) * width[1],
+                              lo.z + (double(c / (size_t(nx) * ny)) + 0.5) * width[2]};
+    const double cell_diag =
+        sqrt(width[0] * width[0] + width[1] * width[1] + width[2] * width[2]);
+    const double u = 5.9604644775390625e-8;  // 2^-24
+    const double q_error = 4.0 * u * fmax(double(nx), fmax(double(ny), double(nz)));
     double p[4][3], d2 = 0.0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -3713,12 +3726,13 @@ hipError_t launch_value_ranges(const KVolume &v, float *ranges, hipStream_t s) {
 size_t scene_lds_size(const KScene &sc) { return scene_lds_bytes(sc); }
 
 hipError_t launch_tet_planes(const uint32_t *start, const float4 *recs, const float lo[3],
-                             const float inv_cell[3], const int dims[3], uint4 *planes,
-                             hipStream_t s) {
-  const size_t cells = size_t(dims[0]) * dims[1] * dims[2];
-  hipLaunchKernelGGL(k_tet_planes, dim3(unsigned((cells + 255) / 256)), dim3(256), 0, s, start,
-                     recs, mk(lo[0], lo[1], lo[2]), mk(inv_cell[0], inv_cell[1], inv_cell[2]),
-                     dims[0], dims[1], dims[2], planes);
+                             const float inv_cell[3], const int dims[3], size_t entries,
+                             uint4 *planes, hipStream_t s) {
+  if (entries == 0) return hipSuccess;
+  const size_t blocks = std::min<size_t>((entries + 255) / 256, 1 << 20);
+  hipLaunchKernelGGL(k_tet_planes, dim3(unsigned(blocks)), dim3(256), 0, s, start, recs,
+                     mk(lo[0], lo[1], lo[2]), mk(inv_cell[0], inv_cell[1], inv_cell[2]), dims[0],
+                     dims[1], dims[2], planes);
   return hipGetLastError();
 }
 

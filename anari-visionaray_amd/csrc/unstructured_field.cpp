@@ -170,7 +170,8 @@ int vrt_unstructured_create(vrt_context ctx, const float *pos, const float *vdat
   if (e == hipSuccess)
     e = hipMemcpyAsync(h->tets, tets.data(), tet_bytes, hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess)
-    e = launch_tet_planes(h->start, h->recs, h->lo, h->inv_cell, h->dims, h->planes, ctx->stream);
+    e = launch_tet_planes(h->start, h->recs, h->lo, h->inv_cell, h->dims, h->entries, h->planes,
+                          ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);  // host copies go out of scope
   if (e != hipSuccess) return cleanup(e, "unstructured field upload");
   h->device_bytes = start_bytes + rec_bytes + rec_bytes / 2 + cell_bytes + tet_bytes;
