@@ -94,7 +94,7 @@ struct KVolume {
   // tetrahedron {bbox min, value min}, {bbox max, value max}
   const uint32_t *ug_start;
   const float4 *ug_recs;
-  const uint4 *ug_planes;  // per list entry: four face planes, 16 halfs (k_tet_planes)
+  const uint4 *ug_planes;  // per list entry: four face planes, 16 halfs (k_tet_planes), or null
   const uint32_t *ug_cell;  // per list entry: primitive id (ANARI cell index)
   const float4 *ug_tets;
   uint32_t ug_num_tets;

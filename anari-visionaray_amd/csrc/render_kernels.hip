@@ -447,6 +447,7 @@ constexpr int kTetBatch = 4;
 // bit k: entry i + k (< e) may contain the point at q, its position relative
 // to the cell's centre in cell widths
 __device__ inline uint32_t tet_candidates(const KVolume &v, uint32_t i, uint32_t e, f3 q) {
+  if (!v.ug_planes) return (2u << min(e - i - 1u, uint32_t(kTetBatch) - 1u)) - 1u;  // all
   uint4 r[2 * kTetBatch];
 #pragma unroll
   for (int k = 0; k < kTetBatch; ++k) {

@@ -157,10 +157,15 @@ int vrt_unstructured_create(vrt_context ctx, const float *pos, const float *vdat
                cell_bytes = rec_cell.size() * 4, tet_bytes = tets.size() * sizeof(float4);
   hipError_t e = hipMalloc(&h->start, start_bytes);
   if (e == hipSuccess) e = hipMalloc(&h->recs, std::max<size_t>(rec_bytes, 64));
-  if (e == hipSuccess) e = hipMalloc(&h->planes, std::max<size_t>(rec_bytes / 2, 64));
   if (e == hipSuccess) e = hipMalloc(&h->rec_cell, std::max<size_t>(cell_bytes, 4));
   if (e == hipSuccess) e = hipMalloc(&h->tets, tet_bytes);
   if (e != hipSuccess) return cleanup(e, "unstructured field allocation");
+  // the planes only save the search exact tests: a field that fills the device
+  // does without
+  if (hipMalloc(&h->planes, std::max<size_t>(rec_bytes / 2, 64)) != hipSuccess) {
+    (void)hipGetLastError();
+    h->planes = nullptr;
+  }
   e = hipMemcpyAsync(h->start, g.start.data(), start_bytes, hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess && rec_bytes)
     e = hipMemcpyAsync(h->recs, g.recs.data(), rec_bytes, hipMemcpyHostToDevice, ctx->stream);
@@ -169,12 +174,13 @@ int vrt_unstructured_create(vrt_context ctx, const float *pos, const float *vdat
                        ctx->stream);
   if (e == hipSuccess)
     e = hipMemcpyAsync(h->tets, tets.data(), tet_bytes, hipMemcpyHostToDevice, ctx->stream);
-  if (e == hipSuccess)
+  if (e == hipSuccess && h->planes)
     e = launch_tet_planes(h->start, h->recs, h->lo, h->inv_cell, h->dims, h->entries, h->planes,
                           ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);  // host copies go out of scope
   if (e != hipSuccess) return cleanup(e, "unstructured field upload");
-  h->device_bytes = start_bytes + rec_bytes + rec_bytes / 2 + cell_bytes + tet_bytes;
+  h->device_bytes =
+      start_bytes + rec_bytes + (h->planes ? rec_bytes / 2 : 0) + cell_bytes + tet_bytes;
   *out = h;
   return VRT_OK;
 }
