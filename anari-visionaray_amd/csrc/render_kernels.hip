@@ -759,6 +759,11 @@ __device__ inline void cswap(float &ta, int &na, float &tb, int &nb) {
 // until all lanes have leaves: 6.8, 5.5, 5.2, 5.5, 5.7, 6.5 ms).
 constexpr int kWalkShare = 3;
 
+// ORDERED: a leaf's triangles are tested in ascending order, so that an any-hit
+// query returns the first one met.  The closest hit, and whether there is any,
+// do not depend on the order; without it the renderers' loop keeps one register
+// less (ray caster, shaded, a mesh in a NanoVDB cloud: 6.39 -> 6.07 ms).
+template <bool ORDERED = false>
 __device__ inline bool bvh_hit(const KSurface &S, const KRay &r, bool any, float &tbest,
                                int &prim, uint32_t &rec, int2 *lst,
                                const float4 *lnodes = nullptr, int lds_nodes = 0) {
@@ -859,19 +864,22 @@ __device__ inline bool bvh_hit(const KSurface &S, const KRay &r, bool any, float
         node = -2;  // pop once the leaves are tested
       }
     } while (counts == 0u && node >= 0 && __popcll(__ballot(true)) * kWalkShare >= lanes0);
-    // the leaves' triangles, in one loop for all four children, each leaf's in
-    // ascending order (any-hit calls return the first one met)
-    uint32_t q0 = 0;
-    uint32_t left = 0;
-    while ((counts | left) != 0u) {
-      if (left == 0u) {
+    // the leaves' triangles, in one loop for all four children
+    uint32_t next = 0, left = 0;
+    while (counts != 0u || (ORDERED && left != 0u)) {
+      uint32_t k;
+      if (!ORDERED || left == 0u) {
         const int c = (__ffs(int(counts)) - 1) >> 3;
-        q0 = uint32_t(c == 0 ? leaf[0] : c == 1 ? leaf[1] : c == 2 ? leaf[2] : leaf[3]);
+        next = uint32_t(c == 0 ? leaf[0] : c == 1 ? leaf[1] : c == 2 ? leaf[2] : leaf[3]);
         left = (counts >> (8 * c)) & 255u;
-        counts &= ~(255u << (8 * c));
+        counts -= ORDERED ? left << (8 * c) : 1u << (8 * c);
       }
-      const uint32_t k = q0++;
-      --left;
+      if constexpr (ORDERED) {
+        k = next++;
+        --left;
+      } else {
+        k = next + left - 1u;
+      }
       const float4 *q = S.tris + 3 * size_t(k);
       const float4 a = q[0], b = q[1], d = q[2];
       float t, u, v;
@@ -900,6 +908,7 @@ __device__ inline bool bvh_hit(const KSurface &S, const KRay &r, bool any, float
 // (`found_before`: a surface hit at tbest keeps ties), else when strictly
 // closer, or equally close on an instance of lower index.  Returns whether
 // an instance was hit; `slot` is its position in T.inst.
+template <bool ORDERED = false>
 __device__ inline bool tls_hit(const KTls &T, const KRay &r, bool any, bool found_before,
                                float &tbest, int &slot, int &prim, uint32_t &rec, int2 *lst) {
   f3 inv;
@@ -956,7 +965,7 @@ __device__ inline bool tls_hit(const KTls &T, const KRay &r, bool any, bool foun
         float t = tbest;
         int p = -1;
         uint32_t rc = 0;
-        if (!bvh_hit(S, lr, any, t, p, rc, lst)) continue;
+        if (!bvh_hit<ORDERED>(S, lr, any, t, p, rc, lst)) continue;
         if ((found_before || found) && !(t < tbest || (found && t == tbest && I.index < best_index)))
           continue;
         found = true;
@@ -3412,7 +3421,7 @@ __global__ void __launch_bounds__(256)
     float t = best;
     int p = -1;
     uint32_t rec;
-    if (bvh_hit(sc.surf[s], ray, any != 0, t, p, rec, s_bstack + threadIdx.x,
+    if (bvh_hit<true>(sc.surf[s], ray, any != 0, t, p, rec, s_bstack + threadIdx.x,
                 lnodes + sc.staged[s].lds_first, sc.staged[s].lds_nodes)) {
       hit = true;
       best = t;
@@ -3424,7 +3433,7 @@ __global__ void __launch_bounds__(256)
     float t = best;
     int slot = -1, p = -1;
     uint32_t rec;
-    if (tls_hit(sc.tls, ray, any != 0, hit, t, slot, p, rec, s_bstack + threadIdx.x)) {
+    if (tls_hit<true>(sc.tls, ray, any != 0, hit, t, slot, p, rec, s_bstack + threadIdx.x)) {
       hit = true;
       best = t;
       prim = p;
