@@ -302,7 +302,7 @@ __device__ inline float sample_structured(const KVolume &v, f3 P) {
 // what counts is their number and the instructions between them: with the
 // tree's own 8^3 leaves behind a top table and blocks (3 dependent reads, and
 // a slot comparison, look-up and branch for each of 7 taps) the cloud 320^3
-// at 1080p took 11.3 ms a frame, now 5.9 ms.
+// at 1080p took 11.3 ms a frame, with records 5.9 ms (4.5 with the walk below).
 // ---------------------------------------------------------------------------
 // entry of the 8^3 slot (sx, sy, sz) (voxel index >> 3): >= 0 record,
 // kNvTreeEntry or -1 - constant index
@@ -1196,13 +1196,17 @@ __device__ inline bool trav_advance(const KVolume &v, Trav &T) {
 // tetrahedra at 1919x1079) and the structured fetch (1, 2, 3, 4, 8 steps:
 // 0.96, 0.84, 0.81, 0.78, 0.87 ms for fBm 512^3 at 1080p).  A NanoVDB lookup
 // (one table read, mostly of a short walk) costs about as much as a step (1,
-// 2, 3, 4: 4.9, 5.4, 5.6, 5.7 ms for the cloud 320^3 at 1080p).
+// 2, 3, 4: 4.9, 5.4, 5.6, 5.7 ms for one view of the cloud 320^3 at 1080p).  Kernels
+// for any field take 2: 1 is 13-20 % slower where there are tetrahedra, 4 is
+// 8-12 % faster there and 5-8 % slower with a NanoVDB field.
 template <int FIELD>
 constexpr int kFreeSteps = FIELD == kNanovdbField ? 1 : FIELD == kTetsField ? 6
                            : FIELD == kAnyField   ? 2 : 4;
 // Ratio tracking looks up every collision of a ray, not about one, so lanes
 // that wait for the others' cells wait more often (2 / 4 steps and claims of 32
-// / 64 pixels below: fBm 192^3 at 1280x720 1.83 / 1.95 ms, 400^3 2.27 / 2.65).
+// / 64 pixels below: fBm 192^3 at 1280x720 1.79 / 1.95 ms, 400^3 2.30 / 2.76).
+// The loop leaves after them rather than counting to a bound of its own, which
+// cost delta tracking 2 % (the loop stays unrolled).
 template <int FIELD>
 constexpr int kRatioSteps = FIELD == kStructuredField ? 2 : kFreeSteps<FIELD>;
 enum WalkTo { kCollision, kWalkOn, kLeft };
@@ -1210,8 +1214,7 @@ enum WalkTo { kCollision, kWalkOn, kLeft };
 template <int FIELD>
 __device__ inline WalkTo trav_next(const KVolume &v, const uint8_t *mb, float mstep, Trav &T,
                                    bool ratio, uint32_t &rs) {
-  const int steps = ratio ? kRatioSteps<FIELD> : kFreeSteps<FIELD>;
-  for (int k = 0; k < steps; ++k) {
+  for (int k = 0; k < kFreeSteps<FIELD>; ++k) {
     if (!T.in_cell) {
       float a0, a1, maj;
       if (T.cells_left < 0) {
@@ -1244,6 +1247,7 @@ __device__ inline WalkTo trav_next(const KVolume &v, const uint8_t *mb, float ms
       T.in_cell = false;  // also on NaN
     }
     if (trav_advance(v, T)) return kLeft;
+    if (kRatioSteps<FIELD> < kFreeSteps<FIELD> && ratio && k + 1 == kRatioSteps<FIELD>) break;
   }
   return kWalkOn;
 }
@@ -3579,12 +3583,12 @@ static PathtraceKernel pathtrace_kernel(const KScene &sc, bool nrc, bool grad) {
 // Pass scheduling of the path tracer (vrt_params.pass_schedule): 1 chains the
 // passes of a bounce (KParams::chain_passes), 2 traces one ray per lane and
 // pass, 3 is 2 with idle lanes refilled only 16 at a time (refill_min).
-// Measured frame times (1 / 2 / 3): fBm 512^3 1.21 / 1.27 / 1.26 ms, mixed
-// surfaces + volume 18.6 / 19.5 / 19.4 ms, NanoVDB cloud 1024^3 3.44 / 3.59 /
-// 3.36 ms (its cache frames 2.82 / 2.83 / 2.77 ms), 2.06 M tetrahedra at
-// 3840x2160 22.0 / 20.5 / 20.9 ms; the default picks per scene: 3 with a
-// NanoVDB field, 2 with a tetrahedral one (and no NanoVDB field), 1
-// otherwise.
+// Measured frame times (1 / 2 / 3): fBm 512^3 0.77 / 0.85 / 0.85 ms, mixed
+// surfaces + volume 10.81 / 11.44 / 11.39 ms, NanoVDB cloud 1024^3 1.51 / 1.46 /
+// 1.44 ms (its cache frames 1.40 / 1.38 / 1.36 ms), 2.06 M tetrahedra at
+// 3840x2160 13.4 / 12.1 / 12.3 ms (cache frames 7.76 / 6.90 / 6.91 ms); the
+// default picks per scene: 3 with a NanoVDB field, 2 with a tetrahedral one
+// (and no NanoVDB field), 1 otherwise.
 int pathtrace_schedule(const KScene &sc) {
   bool nvdb = false, tets = false;
   for (int i = 0; i < sc.num_volumes; ++i) {
