@@ -35,8 +35,9 @@ __host__ __device__ inline float comp(f3 a, int i) { return i == 0 ? a.x : (i ==
 // A NanoVDB tree as two tables (see nanovdb_field.cpp): top table over 128^3
 // regions (>= 0 block index, else -1 - constant) of origin lo (in 128-voxel
 // units) and dims n; blocks of 16^3 slot entries (>= 0 leaf, else -1 -
-// constant); leaf values (512 each; null once the records hold all that
-// lookups read); value range of each slot of the blocks.  In device memory:
+// constant); leaf values (512 each; freed once the records hold all that
+// lookups read: no entry leads to them then); value range of each slot of the
+// blocks.  In device memory:
 // the kernels' arguments hold its address only, as few lookups read it and
 // each word of a volume costs the renderers registers.
 struct KNvTree {

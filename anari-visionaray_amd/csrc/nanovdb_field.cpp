@@ -27,11 +27,11 @@
 // neighbours holds a lower node, else their constant or kNvTreeEntry.
 //
 // Records take 1.4 times the leaves' memory for a solid field, up to 11.5
-// times for leaves that touch no other (8 records of 2,944 B each).  Where they would
-// take more than 64 MB and more than 8 times the tree's tables, or half of the
-// device's free memory, no records are made: every such slot is kNvTreeEntry, a
-// lookup costs what the tree's three dependent reads cost, and the leaves
-// stay.  Else they are freed once the records stand.
+// times for leaves that touch no other (8 records of 2,944 B each).  Where
+// they would take more than 64 MB and more than 8 times the tree's tables, or
+// half of the device's free memory, no records are made: every such slot is
+// kNvTreeEntry, a lookup costs what the tree's three dependent reads cost, and
+// the leaves stay.  Else they are freed once the records stand.
 //
 // Record offsets are those of the 32.7 format (GridData 672 B with the map at
 // 296 and the world bbox at 560; TreeData 64 B; RootData 64 B + 32-B tiles;

@@ -1666,8 +1666,8 @@ __device__ inline float4 light_backdrop(const KScene &sc, const KRay &ray, float
 // the ambient term.  Lights are sampled at P itself, in voxel space, as the
 // reference does.
 template <int FIELD>
-__device__ __forceinline__ f3 gradient_shade(const KScene &sc, const KVolume &v, const KParams &P, f3 Pv,
-                                    f3 viewDir, f3 albedo, uint32_t &rs) {
+__device__ __forceinline__ f3 gradient_shade(const KScene &sc, const KVolume &v, const KParams &P,
+                                             f3 Pv, f3 viewDir, f3 albedo, uint32_t &rs) {
   f3 gn = gradient_normal<FIELD>(v, Pv);
   gn = faceforward(gn, viewDir, gn);
   f3 shaded = mk(0.f);
